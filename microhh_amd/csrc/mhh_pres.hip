@@ -839,70 +839,129 @@ namespace
     };
 
     // Tridiagonal solve per (kx, ky) mode (Pres_2::solve + tdma,
-    // src/pres_2.cxx:266-324, 200-263), one thread per mode marching in k.
-    // The elimination (reciprocal pivots, gamma) depends on the mode only
-    // through lambda and is precomputed per system (Pres_tables::tri_*), so
-    // the sweeps read it instead of writing and re-reading gamma, and divide
-    // nowhere.  TF is the element type of the spectrum, TC the arithmetic type
-    // of the sweep (double in the mixed mode).
-    template<typename TF, typename TC>
-    __device__ __forceinline__ void tdma_g(cplx<TF>* __restrict__ C,
+    // src/pres_2.cxx:266-324, 200-263).  The matrix is real, so the two
+    // components of a mode are two real systems: lane l of a wave owns
+    // component l % 2 of mode l / 2, which are consecutive words of every level
+    // of the spectrum.  The elimination (reciprocal pivots, gamma) depends on
+    // the mode only through lambda and is precomputed per system
+    // (Pres_tables::tri_*): no division in the sweeps.  TF is the element type
+    // of the spectrum, TC the arithmetic type of the sweep (double in the mixed
+    // mode).
+    //
+    // What bounds it: on large grids the bytes (768 x 384 x 256 FP64: 0.57 ms, the
+    // spectrum twice in and out and the two tables), on small ones the chain
+    // over the levels, a multiply-add each if a level's values have arrived.
+    // The loads of TRI_G levels are in flight while the TRI_G before them are
+    // eliminated: 32^3 FP32 7.8 us, 90 x 75 x 60 FP64 15.1, 256 x 192 x 96 mixed
+    // 27, 240 x 180 x 120 FP64 46 (15.5, 36.8, 61.7 and 113 with one level per trip
+    // to memory).  LDSB: the eliminated right-hand side stays in the wave's LDS
+    // column (K x 64 words) for the back substitution, so the spectrum is read
+    // and written once.  Only for columns of at most TRI_LDS bytes, five waves
+    // on a CU: with longer ones too few waves are in flight (1024 x 1024 x 192
+    // mixed, 48 KB: 36.5 against 35.0 ms per step; 768 x 384 x 256 FP64, 128 KB:
+    // 24.3 against 22.0), with shorter ones the saved trip shows (256 x 192 x 96
+    // mixed: 0.94 against 0.96 ms per step).
+    constexpr int TRI_G = 16;
+    constexpr size_t TRI_LDS = 32*1024;
+
+    template<typename TF, typename TC, bool LDSB>
+    __device__ __forceinline__ void tdma_g(TF* __restrict__ C,
                                            const TC* __restrict__ wi, const TC* __restrict__ gam,
                                            const TC* __restrict__ a, const TC* __restrict__ dz2,
                                            int nx, int nsys, Gd g, bool skip_mean, const Bid& bid_)
     {
+        extern __shared__ unsigned char smem_raw[];
+        TF* col = reinterpret_cast<TF*>(smem_raw) + threadIdx.x;    // LDSB: level k at col[64 k]
         const int M = g.jtot, K = g.ktot;
-        const int mode = bid_.x*blockDim.x + threadIdx.x;
         const int nmodes = nx*M;
-        if (mode >= nmodes) return;
-        const int kx = mode / M, ky = mode % M;
+        const int r0 = bid_.x*64 + static_cast<int>(threadIdx.x);
+        const bool active = r0 < 2*nmodes;
+        const int r = active ? r0 : 2*nmodes - 1;
+        const int mode = r >> 1;
+        const int kx = mode / M, ky = mode - kx*M;
         const int l = kx*(M/2 + 1) + (ky <= M/2 ? ky : M - ky);
-        const size_t ks = static_cast<size_t>(nmodes), ls = static_cast<size_t>(nsys);
-        if (kx == 0 && ky == 0 && skip_mean)
+        // the mixed mode solves the horizontal mean in FP64 (mean_mode_g)
+        const bool zero = skip_mean && mode == 0;
+        const size_t ks = 2*static_cast<size_t>(nmodes), ls = static_cast<size_t>(nsys);
+        TF* __restrict__ Cr = C + r;
+        const TC* __restrict__ wr = wi + l;
+        const TC* __restrict__ gr = gam + l;
+
+        TF q[TRI_G], qn[TRI_G];
+        TC w[TRI_G], wn[TRI_G];
+        auto load = [&](TF (&qd)[TRI_G], TC (&wd)[TRI_G], int k0) {
+            #pragma unroll
+            for (int m = 0; m < TRI_G; ++m)
+            {
+                const size_t k = static_cast<size_t>(min(k0 + m, K-1));
+                qd[m] = Cr[k*ks];
+                wd[m] = wr[k*ls];
+            }
+        };
+        // forward elimination (src/pres_2.cxx:200-252); the product with a is
+        // rounded on its own
+        load(q, w, 0);
+        TC pr = TC(0);
+        for (int k0 = 0; k0 < K; k0 += TRI_G)
         {
-            // the mixed mode solves the horizontal mean in FP64 (mean_mode_g)
-            for (int k = 0; k < K; ++k) C[k*ks] = cplx<TF>{TF(0), TF(0)};
-            return;
+            load(qn, wn, k0 + TRI_G);
+            #pragma unroll
+            for (int m = 0; m < TRI_G; ++m)
+            {
+                const int k = k0 + m;
+                if (k < K)
+                {
+                    const TC d = ld_const(dz2, k);
+                    const TC x = (k > 0 ? fma(d, TC(q[m]), -mul_rn(ld_const(a, k), pr)) : d*TC(q[m]))*w[m];
+                    if (LDSB) col[64*k] = TF(x);
+                    else if (active) Cr[k*ks] = TF(x);
+                    pr = x;
+                }
+            }
+            #pragma unroll
+            for (int m = 0; m < TRI_G; ++m) { q[m] = qn[m]; w[m] = wn[m]; }
         }
-        // forward elimination (src/pres_2.cxx:200-252)
-        TC px, py;
+        // back substitution (src/pres_2.cxx:254-262) from the top; w[m] holds
+        // gamma of the level above
+        auto loadb = [&](TF (&qd)[TRI_G], TC (&wd)[TRI_G], int kt) {
+            #pragma unroll
+            for (int m = 0; m < TRI_G; ++m)
+            {
+                const int k = max(kt - m, 0);
+                qd[m] = LDSB ? col[64*k] : Cr[k*ks];
+                wd[m] = gr[static_cast<size_t>(min(k + 1, K-1))*ls];
+            }
+        };
+        loadb(q, w, K-1);
+        for (int k0 = K-1; k0 >= 0; k0 -= TRI_G)
         {
-            const cplx<TF> q = C[mode];
-            const TC w0 = wi[l];
-            px = dz2[0]*TC(q.x)*w0; py = dz2[0]*TC(q.y)*w0;
-            C[mode] = cplx<TF>{TF(px), TF(py)};
-        }
-        for (int k = 1; k < K; ++k)
-        {
-            const cplx<TF> q = C[k*ks + mode];
-            const TC wk = wi[k*ls + l];
-            TC qx = dz2[k]*TC(q.x), qy = dz2[k]*TC(q.y);
-            qx -= a[k]*px; qy -= a[k]*py;
-            qx *= wk; qy *= wk;
-            C[k*ks + mode] = cplx<TF>{TF(qx), TF(qy)};
-            px = qx; py = qy;
-        }
-        // back substitution (src/pres_2.cxx:254-262)
-        for (int k = K-2; k >= 0; --k)
-        {
-            const cplx<TF> q = C[k*ks + mode];
-            const TC gk1 = gam[(k+1)*ls + l];
-            TC qx = TC(q.x), qy = TC(q.y);
-            qx -= gk1*px; qy -= gk1*py;
-            C[k*ks + mode] = cplx<TF>{TF(qx), TF(qy)};
-            px = qx; py = qy;
+            // the levels of the next group are written only in their own group
+            loadb(qn, wn, k0 - TRI_G);
+            #pragma unroll
+            for (int m = 0; m < TRI_G; ++m)
+            {
+                const int k = k0 - m;
+                if (k >= 0)
+                {
+                    const TC x = k == K-1 ? pr : fma(-w[m], pr, TC(q[m]));
+                    if (active) Cr[k*ks] = zero ? TF(0) : TF(x);
+                    pr = x;
+                }
+            }
+            #pragma unroll
+            for (int m = 0; m < TRI_G; ++m) { q[m] = qn[m]; w[m] = wn[m]; }
         }
     }
 
-    template<typename TF, typename TC>
+    template<typename TF, typename TC, bool LDSB>
     struct tdma_k
     {
-        static constexpr int NT = 256, MINB = 0;
-        cplx<TF>* C; const TC* wi; const TC* gam; const TC* a; const TC* dz2; int nx; int nsys; Gd g;
+        static constexpr int NT = 64, MINB = 0;
+        TF* C; const TC* wi; const TC* gam; const TC* a; const TC* dz2; int nx; int nsys; Gd g;
         bool skip_mean;
         __device__ __forceinline__ void operator()(const Bid& bid_) const
         {
-            tdma_g<TF, TC>(C, wi, gam, a, dz2, nx, nsys, g, skip_mean, bid_);
+            tdma_g<TF, TC, LDSB>(C, wi, gam, a, dz2, nx, nsys, g, skip_mean, bid_);
         }
     };
 
@@ -1744,6 +1803,24 @@ namespace
         return check_launch(name);
     }
 
+    // Tridiagonal sweep of every mode, one wave per 32 modes.
+    template<typename TF, typename TC>
+    int tdma(mhh_ctx* c, cplx<TF>* C, const Pres_tables<TC>& t, int nx, bool skip_mean)
+    {
+        const Gd& g = c->gd;
+        const int nb = (2*nx*g.jtot + 63)/64;
+        const size_t lds = sizeof(TF)*64*static_cast<size_t>(g.ktot);
+        {
+            mhh::Timer _t(c, "tdma");
+            TF* Cr = reinterpret_cast<TF*>(C);
+            if (lds <= TRI_LDS)
+                launch(c, tdma_k<TF, TC, true>{Cr, t.tri_wi, t.tri_gam, t.a, t.dz2, nx, t.nsys, g, skip_mean}, nb, 64, lds);
+            else
+                launch(c, tdma_k<TF, TC, false>{Cr, t.tri_wi, t.tri_gam, t.a, t.dz2, nx, t.nsys, g, skip_mean}, nb, 64);
+        }
+        return check_launch("tdma");
+    }
+
     // Fused y transforms and tridiagonal sweep (jtot = 64 R, R = 2, 4, 8).
     template<typename TF, typename TC, int R>
     void launch_ytri(mhh_ctx* c, cplx<TF>* C, const double2* twy, const Pres_tables<TC>& d, int nx, bool skip_mean,
@@ -1958,23 +2035,13 @@ namespace
         else
             MHH_CHECK(fft_y<TF>(c, C, py, t.twy, -1, nrows, "fft_y_fwd"));
         // 4. tridiagonal per mode
+        if constexpr (std::is_same<TF, float>::value)
         {
-            const int nmodes = nx*M;
-            if (c->mixed)
-            {
-                const Pres_tables<double>& d = c->td;
-                mhh::Timer _t(c, "tdma");
-                launch(c, tdma_k<TF, double>{C, d.tri_wi, d.tri_gam, d.a, d.dz2,
-                        nx, d.nsys, g, true}, (nmodes + 255)/256, 256);
-            }
-            else
-            {
-                mhh::Timer _t(c, "tdma");
-                launch(c, tdma_k<TF, TF>{C, t.tri_wi, t.tri_gam, t.a, t.dz2,
-                        nx, t.nsys, g, false}, (nmodes + 255)/256, 256);
-            }
-            MHH_CHECK(check_launch("tdma"));
+            if (c->mixed) MHH_CHECK((tdma<TF, double>(c, C, c->td, nx, true)));
+            else MHH_CHECK((tdma<TF, TF>(c, C, t, nx, false)));
         }
+        else
+            MHH_CHECK((tdma<TF, TF>(c, C, t, nx, false)));
         // 5. inverse y transform (divides by jtot)
         if constexpr (std::is_same<TF, float>::value)
         {
