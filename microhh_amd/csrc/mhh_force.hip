@@ -10,21 +10,39 @@ namespace
     using namespace mhh;
 
     // The dz-weighted volume means of u and ut (Field3d_operators::calc_mean,
-    // src/field3d_operators.cxx:134-155) from their plane means, and the body
-    // force (uflux - u_mean - utrans)/dt - ut_mean, in FP64 by one block.
-    __global__ void __launch_bounds__(64) fixed_flux_force_g(double* __restrict__ buf, const double* __restrict__ dz,
-                                                           double uflux, double utrans, double dti, double zsize,
-                                                           int kstart, int kend, int kcells)
+    // src/field3d_operators.cxx:134-155) from their partial plane sums, and the
+    // body force (uflux - u_mean - utrans)/dt - ut_mean, in FP64 by one block:
+    // a thread takes every FT-th level, the block folds the shares.
+    constexpr int FT = 256;
+
+    __global__ void __launch_bounds__(FT) fixed_flux_force_g(const double* __restrict__ part, double* __restrict__ fbody,
+                                                             const double* __restrict__ dz, int nchunk, int nk,
+                                                             double npoints, double uflux, double utrans, double dti,
+                                                             double zsize)
     {
-        if (threadIdx.x != 0) return;
-        double su = 0., st = 0.;
-        for (int k = kstart; k < kend; ++k)
+        __shared__ double su[FT], st[FT];
+        const int tid = threadIdx.x;
+        double au = 0., at = 0.;
+        for (int k = tid; k < nk; k += FT)
         {
-            su += buf[k]*dz[k];
-            st += buf[kcells + k]*dz[k];
+            double pu = 0., pt = 0.;
+            for (int q = 0; q < nchunk; ++q)
+            {
+                pu += part[static_cast<size_t>(k)*nchunk + q];
+                pt += part[static_cast<size_t>(nk + k)*nchunk + q];
+            }
+            au += (pu/npoints)*dz[k];
+            at += (pt/npoints)*dz[k];
         }
-        const double u_mean = su / zsize, ut_mean = st / zsize;
-        buf[2*kcells] = (uflux - u_mean - utrans)*dti - ut_mean;
+        su[tid] = au; st[tid] = at;
+        __syncthreads();
+        for (int w = FT/2; w > 0; w >>= 1)
+        {
+            if (tid < w) { su[tid] += su[tid + w]; st[tid] += st[tid + w]; }
+            __syncthreads();
+        }
+        if (tid == 0)
+            *fbody = (uflux - su[0]/zsize - utrans)*dti - st[0]/zsize;
     }
 
     template<typename TF>
@@ -41,20 +59,24 @@ namespace
     int fixed_flux(mhh_ctx* c, double uflux, double utrans, double dt)
     {
         const Gd& g = c->gd;
+        const int nchunk = plane_chunks(g);
         if (!c->force_buf)
         {
-            MHH_CHECK(check_hip(hipMalloc(&c->force_buf, sizeof(double)*(2*g.kcells + 1)), "hipMalloc(force)"));
+            MHH_CHECK(check_hip(hipMalloc(&c->force_buf, sizeof(double)*(1 + 2*static_cast<size_t>(g.ktot)*nchunk)),
+                                "hipMalloc(force)"));
             MHH_CHECK(check_hip(hipMalloc(&c->force_dz, sizeof(double)*g.kcells), "hipMalloc(force)"));
             MHH_CHECK(check_hip(hipMemcpy(c->force_dz, c->h_dz.data(), sizeof(double)*g.kcells,
                                           hipMemcpyHostToDevice), "hipMemcpy(force)"));
         }
-        MHH_CHECK(mean_profile<TF>(c, static_cast<const TF*>(c->f.u), c->force_buf));
-        MHH_CHECK(mean_profile<TF>(c, static_cast<const TF*>(c->f.ut), c->force_buf + g.kcells));
         mhh::Timer _t(c, "force");
-        fixed_flux_force_g<<<1, 64, 0, c->stream>>>(c->force_buf, c->force_dz, uflux, utrans, 1./dt,
-                                                    c->h_zh[g.kend], g.kstart, g.kend, g.kcells);
+        double* part = c->force_buf + 1;
+        MHH_CHECK(plane_sums<TF>(c, static_cast<const TF*>(c->f.u), static_cast<const TF*>(c->f.ut), g.kstart, g.ktot,
+                                 part));
+        fixed_flux_force_g<<<1, FT, 0, c->stream>>>(part, c->force_buf, c->force_dz + g.kstart, nchunk, g.ktot,
+                                                    static_cast<double>(g.itot)*g.jtot, uflux, utrans, 1./dt,
+                                                    c->h_zh[g.kend]);
         add_force_g<TF><<<grid3(g, g.kstart, g.kend), dim3(BX, BY), 0, c->stream>>>(
-                static_cast<TF*>(c->f.ut), c->force_buf + 2*g.kcells, g);
+                static_cast<TF*>(c->f.ut), c->force_buf, g);
         return check_launch("force");
     }
 }

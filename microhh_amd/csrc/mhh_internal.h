@@ -152,8 +152,9 @@ struct mhh_ctx
     double mlen_cs = -1.;
     double* mlen_d = nullptr;
     float* mlen_f = nullptr;
-    // Fixed-flux forcing (mhh_force.hip): plane means of u and ut and the
-    // body force (2 kcells + 1), and dz (kcells), allocated on first use.
+    // Fixed-flux forcing (mhh_force.hip): the body force and the partial
+    // plane sums of u and ut (1 + 2 ktot plane_chunks), and dz (kcells),
+    // allocated on first use.
     double* force_buf = nullptr;
     double* force_dz = nullptr;
     // Surface layer and buffer sponge (mhh_surface.hip), when initialised.
@@ -288,10 +289,15 @@ namespace mhh
     // Surface layer and buffer state (mhh_surface.hip).
     void surface_free(mhh_ctx* ctx);
 
-    // Horizontal mean of every level (kcells values, FP64 sums over the
-    // interior, src/field3d_operators.cxx:46-66) into a device array
-    // (mhh_stats.hip).
-    template<typename TF> int mean_profile(mhh_ctx* c, const TF* fld, double* prof);
+    // Plane sums and means (mhh_stats.hip), FP64 sums over the interior in a
+    // fixed order.  plane_sums: partial sums of the levels k0 .. k0+nk-1 of a
+    // and, unless null, b, part[(field*nk + level)*plane_chunks + chunk].
+    // mean_profile: the horizontal mean of every level (kcells values,
+    // src/field3d_operators.cxx:46-66) into the device array prof; part:
+    // kcells*plane_chunks values of scratch.
+    int plane_chunks(const Gd& g);
+    template<typename TF> int plane_sums(mhh_ctx* c, const TF* a, const TF* b, int k0, int nk, double* part);
+    template<typename TF> int mean_profile(mhh_ctx* c, const TF* fld, double* part, double* prof);
 }
 
 #define MHH_CHECK(call) do { int _rc = (call); if (_rc) return _rc; } while (0)

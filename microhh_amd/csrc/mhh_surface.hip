@@ -32,6 +32,7 @@ struct mhh_buffer_state
     int kb = 0, kbh = 0;             // first buffer level of the cell centres and of the faces
     int ndamped = 0;                 // u, v, w and the first ndamped-3 scalars
     double* prof = nullptr;          // (3 + MHH_MAX_SCALARS) x kcells reference profiles (FP64)
+    double* part = nullptr;          // swupdate: partial plane sums of one field
     void* sig_c = nullptr;           // kcells: sigma ((z - zstart)/(zsize - zstart))^beta, 0 below the buffer
     void* sig_h = nullptr;           // the same at the half levels (w)
 };
@@ -696,6 +697,9 @@ namespace
             }
         }
         MHH_CHECK(check_hip(hipMalloc(&b->prof, sizeof(double)*np), "hipMalloc(buffer)"));
+        if (d.swupdate)
+            MHH_CHECK(check_hip(hipMalloc(&b->part, sizeof(double)*static_cast<size_t>(g.kcells)*plane_chunks(g)),
+                                "hipMalloc(buffer)"));
         return check_hip(hipMemcpy(b->prof, prof.data(), sizeof(double)*np, hipMemcpyHostToDevice), "hipMemcpy");
     }
 
@@ -716,7 +720,7 @@ namespace
         }
         if (b.desc.swupdate)
             for (int q = 0; q < b.ndamped; ++q)
-                MHH_CHECK(mean_profile<TF>(c, fl.a[q], b.prof + static_cast<size_t>(q)*g.kcells));
+                MHH_CHECK(mean_profile<TF>(c, fl.a[q], b.part, b.prof + static_cast<size_t>(q)*g.kcells));
         const int kfirst = std::min(b.kb, b.kbh);
         const int ntx = (g.itot + BX - 1)/BX, nty = (g.jtot + BY - 1)/BY;
         mhh::Timer _t(c, "buffer");
@@ -745,6 +749,7 @@ namespace mhh
         {
             mhh_buffer_state* b = c->buf;
             if (b->prof) (void)hipFree(b->prof);
+            if (b->part) (void)hipFree(b->part);
             if (b->sig_c) (void)hipFree(b->sig_c);
             if (b->sig_h) (void)hipFree(b->sig_h);
             delete b;
