@@ -15,8 +15,11 @@
 // consecutive modes with consecutive threads.  The x transforms transpose
 // through LDS to write/read 2*RB consecutive j values per kx.
 //
-// FFT: Stockham autosort, radix 4/2/3/5 passes ping-ponging between two LDS
-// buffers, one 64-wide wavefront per row, twiddles from a host-computed table.
+// FFT: Stockham autosort with twiddles from a host-computed table: a wave per row
+// for 128, 256 and 512 points (here), lane groups for the other lengths in FP64
+// and the mixed mode (mhh_rowfft.hip), DFT-as-GEMM for 1024 in the mixed mode
+// (mhh_dft.hip), and the general engine of mhh_fft.h for plain FP32 and the few
+// lengths that have no lane-group plan.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -1765,8 +1768,23 @@ namespace
         t = Pres_tables<TF>();
     }
 
+    // Calls f with the plan's engine of the general kernels.  FP64 comes here
+    // only for lengths without a lane-group plan (1, 686, 882 and some above
+    // 1024), none of which the in-place engines take (1 has no pass).
+    template<typename TF, typename F>
+    void with_engine(const Plan& p, F f)
+    {
+        if constexpr (std::is_same<TF, float>::value)
+        {
+            if (p.engine == FFT_FAST) return f(std::integral_constant<int, FFT_FAST>{});
+            if (p.engine == FFT_FAST_WIDE) return f(std::integral_constant<int, FFT_FAST_WIDE>{});
+        }
+        f(std::integral_constant<int, FFT_PINGPONG>{});
+    }
+
     // y transform of nrows contiguous rows: the wave-per-row kernel for n = 128,
-    // 256 and 512, the general engine otherwise.
+    // 256 and 512, lane groups where there is a plan, the general engine
+    // otherwise.
     template<typename TF, int R>
     void launch_fft_y_wave(mhh_ctx* c, cplx<TF>* C, const double* tw, int sign, int nrows)
     {
@@ -1780,6 +1798,8 @@ namespace
     template<typename TF>
     int fft_y(mhh_ctx* c, cplx<TF>* C, const Plan& py, const double* tw, int sign, int nrows, const char* name)
     {
+        if ((c->fft_generic || (py.n != 128 && py.n != 256 && py.n != 512)) && c->row_py.n)
+            return row_y<TF, cplx<TF>>(c, C, tw, sign, nrows, name);
         {
             mhh::Timer _t(c, name);
             if (!c->fft_generic && py.n == 512)      launch_fft_y_wave<TF, 8>(c, C, tw, sign, nrows);
@@ -1791,13 +1811,9 @@ namespace
                 const size_t ldsy = lds_bytes(py, RBy, sizeof(cplx<TF>));
                 const auto* t2 = reinterpret_cast<const double2*>(tw);
                 const dim3 grd((nrows + RBy - 1)/RBy), blk(64, RBy);
-                switch (py.engine)
-                {
-                    case FFT_FAST: launch(c, fft_y_k<TF, FFT_FAST>{C, py, t2, sign, nrows, RBy}, grd, blk, ldsy); break;
-                    case FFT_FAST_WIDE:
-                        launch(c, fft_y_k<TF, FFT_FAST_WIDE>{C, py, t2, sign, nrows, RBy}, grd, blk, ldsy); break;
-                    default: launch(c, fft_y_k<TF, FFT_PINGPONG>{C, py, t2, sign, nrows, RBy}, grd, blk, ldsy); break;
-                }
+                with_engine<TF>(py, [&](auto e) {
+                    launch(c, fft_y_k<TF, decltype(e)::value>{C, py, t2, sign, nrows, RBy}, grd, blk, ldsy);
+                });
             }
         }
         return check_launch(name);
@@ -1925,13 +1941,9 @@ namespace
           const auto* t2 = reinterpret_cast<const double2*>(t.twx);
           const double* pm = c->mixed ? c->pm_mean : nullptr;
           const dim3 blk(64, RB);
-          switch (px.engine)
-          {
-              case FFT_FAST: launch(c, fft_x_fwd_k<TF, FFT_FAST>{P, C, px, t2, RB, g, pm, pin, fuse_in}, grd, blk, lds); break;
-              case FFT_FAST_WIDE:
-                  launch(c, fft_x_fwd_k<TF, FFT_FAST_WIDE>{P, C, px, t2, RB, g, pm, pin, fuse_in}, grd, blk, lds); break;
-              default: launch(c, fft_x_fwd_k<TF, FFT_PINGPONG>{P, C, px, t2, RB, g, pm, pin, fuse_in}, grd, blk, lds);
-          } }
+          with_engine<TF>(px, [&](auto e) {
+              launch(c, fft_x_fwd_k<TF, decltype(e)::value>{P, C, px, t2, RB, g, pm, pin, fuse_in}, grd, blk, lds);
+          }); }
         return check_launch("fft_x_fwd");
     }
 
@@ -1963,10 +1975,13 @@ namespace
                          p.dzi, p.rhoref, p.rhorefh, dxi, dyi, dti};
         const bool xwave = !c->fft_generic && (N == 128 || N == 256 || N == 512) && M % (2*xwaves<TF>()) == 0
                         && g.igc <= 32;
-        // The wave x transform evaluates the right-hand side itself (and, in
-        // the mixed mode, the FP64 plane sums); the general engine does so
-        // except in the mixed mode, whose plane means come first.
-        const int fuse_in = (xwave || !c->mixed) ? 1 : 0;
+        const bool xdft = !xwave && dft_applies(c, N);
+        const bool xrow = !xwave && !xdft && c->row_px.n;
+        // The wave and lane-group x transforms evaluate the right-hand side
+        // themselves (and, in the mixed mode, the FP64 plane sums); the general
+        // engine does so except in the mixed mode, whose plane means come
+        // first, as they do for the matrix-core transform.
+        const int fuse_in = (xwave || xrow || !c->mixed) ? 1 : 0;
         const Pres_tables<double>& d = c->td;
         const size_t mm_lds = sizeof(double)*K;
         if (!fuse_in)
@@ -1989,23 +2004,23 @@ namespace
         const bool ywave = !c->fft_generic && !c->ytri_split && (M == 128 || M == 256 || M == 512);
         const int packed = xwave && ywave ? 1 : 0;
         // 2. forward x transform
-        if (xwave)
+        if (xwave || xrow)
         {
             const int mode = c->mixed ? 3 : 2;
-            MHH_CHECK(fft_x_fwd_wave<TF>(c, P, C, t.twx, mode, p, dxi, dyi, dti, "pres_in_fft_x", packed));
+            if (xwave) MHH_CHECK(fft_x_fwd_wave<TF>(c, P, C, t.twx, mode, p, dxi, dyi, dti, "pres_in_fft_x", packed));
+            else MHH_CHECK((row_x_fwd<TF, T>(c, C, t.twx, c->mixed ? c->pm_part : nullptr, p, dxi, dyi, dti)));
             if (c->mixed)
             {
-                { mhh::Timer _t(c, "pres_mean"); launch(c, mean_mode_k{c->pm_part, M/(2*xwaves<TF>()), c->pm_mean,
+                const int nparts = xwave ? M/(2*xwaves<TF>()) : row_x_nparts(c);
+                { mhh::Timer _t(c, "pres_mean"); launch(c, mean_mode_k{c->pm_part, nparts, c->pm_mean,
                         c->pbar, c->dpbar, d.a, d.dz2, c->pm_coef, 1./(double(N)*double(M)), g}, 1, 256, mm_lds); }
                 MHH_CHECK(check_launch("mean_mode"));
             }
         }
         else if constexpr (std::is_same<TF, float>::value)
         {
-            if (!fuse_in && dft_applies(c, N))
-                MHH_CHECK(dft_x_fwd(c, P, C, c->pm_mean));
-            else
-                MHH_CHECK(fft_x_fwd_general<TF>(c, P, C, px, t, pin, fuse_in));
+            if (xdft) MHH_CHECK(dft_x_fwd(c, P, C, c->pm_mean));
+            else MHH_CHECK(fft_x_fwd_general<TF>(c, P, C, px, t, pin, fuse_in));
         }
         else
             MHH_CHECK(fft_x_fwd_general<TF>(c, P, C, px, t, pin, fuse_in));
@@ -2056,10 +2071,11 @@ namespace
             MHH_CHECK(fft_x_bwd_wave<TF>(c, C, P, t.twx, packed));
         else
         {
-            bool done = false;
             if constexpr (std::is_same<TF, float>::value)
-                if (dft_applies(c, N)) { MHH_CHECK(dft_x_bwd(c, C, P)); done = true; }
-            if (!done)
+                if (xdft) MHH_CHECK(dft_x_bwd(c, C, P));
+            if (xrow)
+                MHH_CHECK((row_x_bwd<TF, T>(c, C, P, t.twx)));
+            else if (!xdft)
             {
                 const int RB = rows_per_block(px, sizeof(T));
                 const dim3 grd((M + 2*RB - 1)/(2*RB), K);
@@ -2067,12 +2083,9 @@ namespace
                 const auto* t2 = reinterpret_cast<const double2*>(t.twx);
                 mhh::Timer _t(c, "fft_x_bwd");
                 const dim3 blk(64, RB);
-                switch (px.engine)
-                {
-                    case FFT_FAST: launch(c, fft_x_bwd_k<TF, FFT_FAST>{C, P, px, t2, RB, g}, grd, blk, lds); break;
-                    case FFT_FAST_WIDE: launch(c, fft_x_bwd_k<TF, FFT_FAST_WIDE>{C, P, px, t2, RB, g}, grd, blk, lds); break;
-                    default: launch(c, fft_x_bwd_k<TF, FFT_PINGPONG>{C, P, px, t2, RB, g}, grd, blk, lds); break;
-                }
+                with_engine<TF>(px, [&](auto e) {
+                    launch(c, fft_x_bwd_k<TF, decltype(e)::value>{C, P, px, t2, RB, g}, grd, blk, lds);
+                });
                 MHH_CHECK(check_launch("fft_x_bwd"));
             }
         }
@@ -2209,12 +2222,14 @@ namespace mhh
         if (c->precision == MHH_FP64 || c->mixed) MHH_CHECK(setup_tables<double>(c, c->td));
         if (c->precision == MHH_FP32) MHH_CHECK(setup_tables<float>(c, c->tf));
         MHH_CHECK(dft_init(c));
+        row_plans_init(c);
         if (c->mixed)
         {
             const size_t K = c->gd.ktot, nk = c->gd.kcells;
             // partial plane sums: PM_CHUNKS per level (plane_sum_g) or one per
-            // block of 8 rows (the wave x transform)
-            const size_t nparts = std::max<size_t>(PM_CHUNKS, (c->gd.jtot + 7)/8);
+            // block of rows (the wave and lane-group x transforms)
+            const size_t nparts = std::max<size_t>({PM_CHUNKS, static_cast<size_t>(c->gd.jtot + 7)/8,
+                                                    static_cast<size_t>(row_x_nparts(c))});
             MHH_CHECK(check_hip(hipMalloc(&c->pm_part, sizeof(double)*K*nparts), "hipMalloc(pm_part)"));
             MHH_CHECK(check_hip(hipMalloc(&c->pm_mean, sizeof(double)*K), "hipMalloc(pm_mean)"));
             MHH_CHECK(check_hip(hipMalloc(&c->pbar, sizeof(double)*nk), "hipMalloc(pbar)"));
