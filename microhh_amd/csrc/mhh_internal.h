@@ -219,12 +219,21 @@ namespace mhh
 
     // Levels per block of the k-marching plane-ring kernels: 64, or fewer
     // on small grids, so that a launch still has about 4 blocks per CU (each
-    // chunk reads a few levels past its ends again; 8 levels is the floor).
-    // The results do not depend on it.
-    inline int march_kchunk(int ntiles_xy, int ktot)
+    // chunk reads a few levels past its ends again; 8 levels is the floor), and
+    // down to 2 levels while the launch has fewer than `least` blocks: a level
+    // costs a block a trip to memory, and reading the ends again costs little
+    // where most of the chip is idle.  least: a block per CU for the tendency
+    // passes, whose chunks begin with a dozen planes (32^3 FP32, 32 blocks of 8 levels:
+    // 27.6 us, 128 of 2: 14.5; but 90 x 75 x 60 FP64, 304 blocks of 8, gains nothing
+    // from 4, and 150 x 100 x 75 FP32, 750 of 8, loses a fifth), four for the
+    // viscosity (32^3 13.5 and 8.5 us, 90 x 75 x 60 17.8 and 13.8).  The results do not depend on it.
+    constexpr int MARCH_LEAST_TEND = 256, MARCH_LEAST_VISC = 1024;
+    inline int march_kchunk(int ntiles_xy, int ktot, int least)
     {
+        auto blocks = [&](int kc) { return static_cast<long>(ntiles_xy)*((ktot + kc - 1)/kc); };
         int kc = 64;
-        while (kc > 8 && static_cast<long>(ntiles_xy)*((ktot + kc - 1)/kc) < 1024) kc /= 2;
+        while (kc > 8 && blocks(kc) < 1024) kc /= 2;
+        while (kc > 2 && blocks(kc) < least) kc /= 2;
         return kc;
     }
 
@@ -232,9 +241,9 @@ namespace mhh
     // merged with the other members', which fill the chip together, so each
     // member marches 32 levels per chunk (64-member ensemble step: 8.63 ms,
     // against 9.19 with 64 levels and 8.87 with 16).
-    inline int march_kchunk(const mhh_ctx* c, int ntiles_xy, int ktot)
+    inline int march_kchunk(const mhh_ctx* c, int ntiles_xy, int ktot, int least)
     {
-        return c->rec ? 32 : march_kchunk(ntiles_xy, ktot);
+        return c->rec ? 32 : march_kchunk(ntiles_xy, ktot, least);
     }
 
     // Max-reductions: each thread folds a chunk of RED_KCHUNK levels of its

@@ -235,7 +235,7 @@ namespace
         a.visc = TF(visc); a.svisc = TF(svisc);
         a.nti = (g.itot + TX - 1)/TX;
         a.ntj = (g.jtot + TY - 1)/TY;
-        a.kchunk = c->tend_kchunk > 0 ? c->tend_kchunk : march_kchunk(c, a.nti*a.ntj, g.ktot);
+        a.kchunk = c->tend_kchunk > 0 ? c->tend_kchunk : march_kchunk(c, a.nti*a.ntj, g.ktot, MARCH_LEAST_TEND);
         a.nkc = (g.ktot + a.kchunk - 1)/a.kchunk;
         const int nblocks = xcd_blocks(a.nti*a.ntj*a.nkc);
         const int ns = c->f.nscalars > 0 ? 1 : 0;

@@ -612,7 +612,7 @@ namespace
         const TF* dpb = c->mixed ? reinterpret_cast<const TF*>(c->dpbar) : nullptr;
         a.nti = (g.itot + VX - 1)/VX;
         a.ntj = (g.jtot + VY - 1)/VY;
-        a.kchunk = c->tend_kchunk > 0 ? c->tend_kchunk : march_kchunk(c, a.nti*a.ntj, g.ktot);
+        a.kchunk = c->tend_kchunk > 0 ? c->tend_kchunk : march_kchunk(c, a.nti*a.ntj, g.ktot, MARCH_LEAST_TEND);
         a.nkc = (g.ktot + a.kchunk - 1)/a.kchunk;
         const int ntiles = a.nti*a.ntj*a.nkc;
         const int nblocks = (ntiles + 7)/8*8;
