@@ -43,6 +43,7 @@ namespace
     constexpr int FW = VX + 2, FH = VY + 2, FN = FW*FH;        // halo-1 planes (evisc)
     constexpr int NQ3 = (QN + TEND_NT - 1)/TEND_NT;
     constexpr int NQ1 = (FN + TEND_NT - 1)/TEND_NT;
+    static_assert(NQ1 == 2 && FN - TEND_NT <= TEND_NT/2, "two rounds, the second for half the waves");
 
     // strain2_acc accessors: the plane ring (u, v at k-1, k, k+1 and w at k,
     // k+1 around the point, QW wide) and global memory.
@@ -304,10 +305,13 @@ namespace
             if (k + 1 < g.kend)
             {
                 const Level<TF> L1 = ld_const(lev, k + 1);
+                // the second round has work for two of the four waves (84 of the
+                // 340 positions): for waves 0 and 1 at even levels and 2 and 3 at
+                // odd ones, so that no SIMD runs both rounds at every level
                 #pragma unroll 1
                 for (int q = 0; q < NQ1; ++q)
                 {
-                    const int idx = tid + q*TEND_NT;
+                    const int idx = q == 0 ? tid : TEND_NT + ((tid + (k & 1)*(TEND_NT/2)) & (TEND_NT - 1));
                     if (idx < FN)
                     {
                         const int pj = idx / FW, pi = idx - pj*FW;
