@@ -1,15 +1,8 @@
-// mhh_fft.h -- complex Stockham FFT of one row in LDS, executed by one
-// 64-lane wavefront, for the spectral pressure solver.
-//
-// Two engines share a Plan:
-//   fast (in place): every pass reads the lane's butterfly inputs into
-//     registers, applies twiddles from an LDS table and a radix-8/4/2/3/5 DFT,
-//     then (after a barrier) writes the outputs back into the same row buffer.
-//     Used when every radix is in {2, 3, 4, 5, 8} and no pass has more than
-//     256 butterflies (<= 4 per lane), i.e. n <= 2048 for powers of two;
-//     lengths whose passes fit 16 complex values per lane (n <= 1024 for
-//     powers of two, 768 = 4 8 8 3) take an instance with half the registers.
-//   ping-pong: the general fallback for any radix up to 13 (two row buffers).
+// mhh_fft.h -- pieces of the complex Stockham FFTs of the spectral pressure
+// solver: complex arithmetic, the factorisation into radices and the DFT codelets
+// of the lane-group engine (mhh_rowfft.h), and the transform of one row in LDS by
+// one wavefront for any radix up to 13 (two row buffers), for the lengths that
+// engine has no plan for.
 // tw[t] = exp(-2 pi i t / n); sign = -1 forward, +1 inverse (unnormalised).
 #pragma once
 
@@ -19,28 +12,12 @@ namespace mhh
 {
     constexpr int FFT_MAXPASS = 16;
     constexpr int FFT_MAXRADIX = 13;
-    constexpr int FFT_MAXB = 4;     // butterflies per lane and pass in the fast engine
-
-    // Butterflies per lane a fast pass of radix r holds in `vals` complex
-    // registers: at most FFT_MAXB, and at most vals/r.
-    __host__ __device__ constexpr int fast_butterflies(int r, int vals)
-    {
-        return vals/r < FFT_MAXB ? vals/r : FFT_MAXB;
-    }
-
-    // The engines, one kernel instance each: the fast engine with 16 complex
-    // values per lane and pass (radix 8: 2 butterflies, 5: 3, else 4), the
-    // same with 32 (4 of every radix; for the lengths above 1024 that need
-    // it, at the cost of registers), and the ping-pong fallback.
-    enum { FFT_FAST = 0, FFT_FAST_WIDE = 1, FFT_PINGPONG = 2 };
-    __host__ __device__ constexpr int engine_vals(int eng) { return eng == FFT_FAST ? 16 : 32; }
 
     struct Plan
     {
         int n;
         int npass;
-        int fast;       // nonzero: an in-place fast engine applies
-        int engine;     // FFT_FAST, FFT_FAST_WIDE or FFT_PINGPONG
+        int fast;       // nonzero: radices 2, 3, 4, 5, 8 and at most 256 butterflies in every pass
         int radix[FFT_MAXPASS];
     };
 
@@ -64,20 +41,15 @@ namespace mhh
                 p.radix[p.npass++] = r; m /= r;
             }
         if (m != 1) return false;
-        p.engine = FFT_FAST;
         for (int q = 0; q < p.npass; ++q)
         {
             const int r = p.radix[q];
-            if (!(r == 2 || r == 3 || r == 4 || r == 5 || r == 8) || n / r > 64*FFT_MAXB)
-                p.engine = FFT_PINGPONG;
-            else if (n / r > 64*fast_butterflies(r, engine_vals(FFT_FAST)) && p.engine == FFT_FAST)
-                p.engine = FFT_FAST_WIDE;
+            if (!(r == 2 || r == 3 || r == 4 || r == 5 || r == 8) || n/r > 256) p.fast = 0;
         }
-        p.fast = p.engine != FFT_PINGPONG;
         return true;
     }
 
-    // LDS layout of rows and of the twiddle table: one unused slot after every
+    // LDS layout of rows and twiddle tables: one unused slot after every
     // 8 complex values, so that the stride-R stores of the early Stockham
     // passes and the strided twiddle reads spread over the LDS banks; rows
     // are an odd number of 16-byte slots apart for the row-crossing loops.
@@ -156,94 +128,7 @@ namespace mhh
         }
     }
 
-    template<typename TF, int R>
-    __device__ __forceinline__ void pass_load(cplx<TF>* v, const cplx<TF>* a, const cplx<TF>* tw,
-                                              int j, int nr, int k, int tstride, int sign)
-    {
-        using T = cplx<TF>;
-        #pragma unroll
-        for (int r = 0; r < R; ++r)
-            v[r] = a[lpad(j + r*nr)];
-        if (k > 0)
-        {
-            #pragma unroll
-            for (int r = 1; r < R; ++r)
-            {
-                T w = tw[lpad(r*k*tstride)];
-                if (sign > 0) w.y = -w.y;
-                v[r] = cmul(v[r], w);
-            }
-        }
-        dft<TF, R>(v, sign);
-    }
-
-    template<typename TF, int R>
-    __device__ __forceinline__ void pass_store(cplx<TF>* a, const cplx<TF>* v, int j, int Ns, int k)
-    {
-        const int idxD = (j / Ns)*Ns*R + k;
-        #pragma unroll
-        for (int r = 0; r < R; ++r)
-            a[lpad(idxD + r*Ns)] = v[r];
-    }
-
-    // Fast engine: in place in row a; tw is the LDS twiddle table of length n;
-    // VALS complex values per lane and pass.  Contains block barriers: every
-    // thread of the block must call it.
-    template<typename TF, int VALS>
-    __device__ void fft_row_inplace(cplx<TF>* a, const cplx<TF>* tw, const Plan& plan, int sign, int lane)
-    {
-        using T = cplx<TF>;
-        const int n = plan.n;
-        int Ns = 1;
-        for (int p = 0; p < plan.npass; ++p)
-        {
-            const int R = plan.radix[p];
-            const int nr = n / R;
-            const int tstride = n / (Ns*R);
-            // butterfly b of radix r in v[b r .. b r + r - 1]; the plan's
-            // engine has room for every pass (fast_butterflies)
-            T v[VALS];
-            #pragma unroll
-            for (int b = 0; b < FFT_MAXB; ++b)
-            {
-                const int j = lane + 64*b;
-                if (j < nr)
-                {
-                    const int k = j % Ns;
-                    switch (R)
-                    {
-                        case 8: if (b < fast_butterflies(8, VALS)) pass_load<TF, 8>(v + 8*b, a, tw, j, nr, k, tstride, sign); break;
-                        case 4: pass_load<TF, 4>(v + 4*b, a, tw, j, nr, k, tstride, sign); break;
-                        case 2: pass_load<TF, 2>(v + 2*b, a, tw, j, nr, k, tstride, sign); break;
-                        case 3: pass_load<TF, 3>(v + 3*b, a, tw, j, nr, k, tstride, sign); break;
-                        default: if (b < fast_butterflies(5, VALS)) pass_load<TF, 5>(v + 5*b, a, tw, j, nr, k, tstride, sign); break;
-                    }
-                }
-            }
-            __syncthreads();
-            #pragma unroll
-            for (int b = 0; b < FFT_MAXB; ++b)
-            {
-                const int j = lane + 64*b;
-                if (j < nr)
-                {
-                    const int k = j % Ns;
-                    switch (R)
-                    {
-                        case 8: if (b < fast_butterflies(8, VALS)) pass_store<TF, 8>(a, v + 8*b, j, Ns, k); break;
-                        case 4: pass_store<TF, 4>(a, v + 4*b, j, Ns, k); break;
-                        case 2: pass_store<TF, 2>(a, v + 2*b, j, Ns, k); break;
-                        case 3: pass_store<TF, 3>(a, v + 3*b, j, Ns, k); break;
-                        default: if (b < fast_butterflies(5, VALS)) pass_store<TF, 5>(a, v + 5*b, j, Ns, k); break;
-                    }
-                }
-            }
-            __syncthreads();
-            Ns *= R;
-        }
-    }
-
-    // Fallback engine: ping-pong between a and b, twiddles from the global
+    // Ping-pong between a and b, twiddles from the global
     // table; returns the buffer holding the result.  Contains block barriers.
     template<typename TF>
     __device__ cplx<TF>* fft_row_pingpong(cplx<TF>* a, cplx<TF>* b, const Plan& plan,
@@ -296,38 +181,6 @@ namespace mhh
         return a;
     }
 
-    // Row FFT through whichever engine the plan allows.  Row layout per block:
-    // fast plans use one padded buffer per row, the fallback two
-    // (a, a + row_half(n)).  Element x of a row lives at index lpad(x).
-    // ENG: the plan's engine; the kernels are instantiated for each, so the
-    // fallback's per-lane arrays (scratch) and the wide engine's registers
-    // stay out of the fast kernels.
-    template<typename TF, int ENG>
-    __device__ __forceinline__ cplx<TF>* fft_row(cplx<TF>* a, const cplx<TF>* tw_lds, const double2* __restrict__ tw_glob,
-                                                 const Plan& plan, int sign, int lane)
-    {
-        if constexpr (ENG == FFT_PINGPONG)
-            return fft_row_pingpong<TF>(a, a + row_half(plan.n), plan, tw_glob, sign, lane);
-        else
-        {
-            fft_row_inplace<TF, engine_vals(ENG)>(a, tw_lds, plan, sign, lane);
-            return a;
-        }
-    }
-
-    // Copy the twiddle table into LDS (all threads of the block participate).
-    template<typename TF>
-    __device__ __forceinline__ void load_twiddles(cplx<TF>* tw_lds, const double2* __restrict__ tw, int n)
-    {
-        const int nthr = blockDim.x*blockDim.y;
-        for (int t = threadIdx.x + blockDim.x*threadIdx.y; t < n; t += nthr)
-        {
-            cplx<TF> w; w.x = TF(tw[t].x); w.y = TF(tw[t].y);
-            tw_lds[lpad(t)] = w;
-        }
-    }
-
-    // Elements per row buffer (complex) for a plan, and of the LDS twiddle table.
-    __host__ __device__ inline int row_elems(const Plan& p) { return p.fast ? row_half(p.n) : 2*row_half(p.n); }
-    __host__ __device__ inline int tw_elems(const Plan& p) { return lpad(p.n - 1) + 1; }
+    // Elements of the two row buffers (complex).
+    __host__ __device__ inline int row_elems(const Plan& p) { return 2*row_half(p.n); }
 }

@@ -93,18 +93,19 @@ namespace mhh
 namespace mhh
 {
     // Plan of a transform by lane groups (mhh_rowfft.h).
-    constexpr int ROW_MAXPASS = 4;
+    constexpr int ROW_MAXPASS = 8;
     struct Row_plan
     {
         int n = 0;                  // 0: no plan
         int npass;
         int lsh;                    // 1 << lsh lanes per row
-        int vals;                   // the kernel instance: ROW_VALS or ROW_VALS_WIDE
+        int vals;                   // the kernel instance: ROW_VALS or ROW_VALS_WIDE values per lane
+        int arith;                  // and its butterflies: ROW_RADIX8 or ROW_DIRECT
         int radix[ROW_MAXPASS];
         int nb[ROW_MAXPASS];        // butterflies n/R
         int ns[ROW_MAXPASS];        // product of the radices before
-        int ts[ROW_MAXPASS];        // twiddle stride n/(Ns R)
-        unsigned int mg[ROW_MAXPASS];   // j/Ns = (j mg) >> 22 for j < 2048
+        int ts[ROW_MAXPASS];        // twiddle stride n/(ns R)
+        unsigned int mg[ROW_MAXPASS];   // j/ns = (j mg) >> 22 for j < 2048
     };
 }
 
@@ -143,10 +144,10 @@ struct mhh_ctx
     // y transforms and tridiagonal sweep as separate passes even where the
     // fused ones apply (a check of the fused kernels).
     bool ytri_split = false;
-    // Plans of the x and y transforms by lane groups (FP64 and mixed mode).
+    // Plans of the x and y transforms by lane groups.
     mhh::Row_plan row_px, row_py;
     // Mixed mode, length 1024: x and y transforms as DFT-as-GEMM on the matrix
-    // cores (mhh_dft.hip) instead of the general engine; tables per context.
+    // cores (mhh_dft.hip) instead of by lane groups; tables per context.
     bool dft_mfma = true;
     int visc_mode = 0;            // the viscosity with the tendencies: 0 by grid size, 1 two passes, 2 one pass
     void* sfc_keep = nullptr;     // du/dz, dv/dz, db/dz kept for the viscosity (three planes)
@@ -304,7 +305,7 @@ namespace mhh
     void pres_free(mhh_ctx* ctx);
 
     // DFT-as-GEMM transforms of length 1024 in the mixed mode (mhh_dft.hip):
-    // whether they replace the general engine for a length n, their tables,
+    // whether they replace the lane groups for a length n, their tables,
     // and the forward x (real rows of P minus the plane mean -> C[k][kx][j]),
     // y (in place on C's rows, sign -1 forward, +1 inverse with 1/jtot) and
     // inverse x (C -> ghosted p with halos, 1/itot) passes.
@@ -315,17 +316,16 @@ namespace mhh
     int dft_y(mhh_ctx* ctx, float2* C, int nrows, int sign);
     int dft_x_bwd(mhh_ctx* ctx, const float2* C, float* p);
 
-    // Transforms by lane groups for lengths without kernels of their own, FP64
-    // and mixed mode (mhh_rowfft.hip): the plans of a context (n = 0 where there
-    // is none); the forward x transform with the right-hand side of the
-    // projection evaluated in it (part, mixed mode: its FP64 sums, row_x_nparts
-    // per level) into C[k][kx][j]; the y transforms in place on C's rows (sign -1
-    // forward, +1 inverse with 1/jtot); the inverse x transform into the ghosted
-    // p with halos, 1/itot.
+    // Transforms by lane groups for lengths without kernels of their own
+    // (mhh_rowfft.hip): the plans of a context (n = 0 where there
+    // is none); the forward x transform of the projection's right-hand side,
+    // evaluated in it or (mixed mode) read from P minus the plane means pm_mean, into
+    // C[k][kx][j]; the y transforms in place on C's rows (sign -1 forward, +1
+    // inverse with 1/jtot); the inverse x transform into the ghosted p with halos,
+    // 1/itot.
     void row_plans_init(mhh_ctx* ctx);
-    int row_x_nparts(const mhh_ctx* ctx);
     template<typename TF, typename T>
-    int row_x_fwd(mhh_ctx* ctx, T* C, const double* tw, double* part, const Prof<TF>& p, TF dxi, TF dyi, TF dti);
+    int row_x_fwd(mhh_ctx* ctx, const TF* P, T* C, const double* tw, const Prof<TF>& p, TF dxi, TF dyi, TF dti);
     template<typename TF, typename T> int row_y(mhh_ctx* ctx, T* C, const double* tw, int sign, int nrows, const char* name);
     template<typename TF, typename T> int row_x_bwd(mhh_ctx* ctx, const T* C, TF* p, const double* tw);
 

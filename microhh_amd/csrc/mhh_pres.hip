@@ -16,10 +16,9 @@
 // through LDS to write/read 2*RB consecutive j values per kx.
 //
 // FFT: Stockham autosort with twiddles from a host-computed table: a wave per row
-// for 128, 256 and 512 points (here), lane groups for the other lengths in FP64
-// and the mixed mode (mhh_rowfft.hip), DFT-as-GEMM for 1024 in the mixed mode
-// (mhh_dft.hip), and the general engine of mhh_fft.h for plain FP32 and the few
-// lengths that have no lane-group plan.
+// for 128, 256 and 512 points (here), lane groups for the other lengths
+// (mhh_rowfft.hip), DFT-as-GEMM for 1024 in the mixed mode (mhh_dft.hip), and the ping-pong engine of mhh_fft.h for the few lengths that have
+// no lane-group plan.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -116,8 +115,6 @@ namespace
     // slot each as (row a, row b); every other kx holds (Xa, Xb) in two slots.
     __device__ __forceinline__ int stage_base(int kx, int n) { return (n & 1) ? 2*kx - 1 : 2*kx; }
 
-    constexpr int MAXQ = 9;   // (n/2 + 1)/64 rounded up for the largest fast plan (n = 1024)
-
     template<typename TF>
     __device__ __forceinline__ void unpack_pair(cplx<TF> z, cplx<TF> c, cplx<TF>& xa, cplx<TF>& xb)
     {
@@ -135,93 +132,56 @@ namespace
         else { const int b = stage_base(kx, n); S[lpad(b)] = xa; S[lpad(b+1)] = xb; }
     }
 
+    // The transforms of the lengths without a lane-group plan.
     // Forward x transform: RB complex rows per block, each packing two real
     // rows of P at level k; writes C[k][kx][j] for kx <= itot/2.
-    template<typename TF, int ENG>
+    template<typename TF>
     __device__ __forceinline__ void fft_x_fwd_g(const TF* __restrict__ P, cplx<TF>* __restrict__ C,
                                                 const Plan& plan, const double2* __restrict__ tw, int RB, Gd g,
                                                 const double* __restrict__ pmean, Pin_args<TF> pin, int fuse_in, const Bid& bid_)
     {
         using T = cplx<TF>;
         extern __shared__ unsigned char smem_raw[];
-        T* tws = reinterpret_cast<T*>(smem_raw);
         const int n = plan.n, nx = n/2 + 1, M = g.jtot, re = row_elems(plan);
-        T* rows = tws + tw_elems(plan);
+        T* rows = reinterpret_cast<T*>(smem_raw);
         const int row = threadIdx.y, lane = threadIdx.x;
         const int k = bid_.y;
         const int j0 = bid_.x*2*RB;              // first real row of the block
         const int ja = j0 + 2*row, jb = ja + 1;
         T* A = rows + row*re;
-        if (plan.fast) load_twiddles<TF>(tws, tw, n);
         const TF* Pk = P + static_cast<size_t>(k)*n*M;
-        if (fuse_in)
+        // mixed mode (pmean): the plane mean is solved separately in FP64
+        const double m = !fuse_in && pmean ? pmean[k] : 0.;
+        for (int x = lane; x < n; x += 64)
         {
-            // the right-hand side evaluated here instead of in pres_in_g
-            for (int x = lane; x < n; x += 64)
+            T z;
+            if (fuse_in)
             {
-                T z;
+                // the right-hand side evaluated here instead of in pres_in_g
                 z.x = (ja < M) ? pres_rhs(pin, x, ja, k, g) : TF(0);
                 z.y = (jb < M) ? pres_rhs(pin, x, jb, k, g) : TF(0);
-                A[lpad(x)] = z;
             }
-        }
-        else if (pmean)
-        {
-            // mixed mode: the plane mean is solved separately in FP64
-            const double m = pmean[k];
-            for (int x = lane; x < n; x += 64)
+            else
             {
-                T z;
                 z.x = (ja < M) ? TF(double(Pk[x + ja*n]) - m) : TF(0);
                 z.y = (jb < M) ? TF(double(Pk[x + jb*n]) - m) : TF(0);
-                A[lpad(x)] = z;
             }
+            A[lpad(x)] = z;
         }
-        else
-            for (int x = lane; x < n; x += 64)
-            {
-                T z;
-                z.x = (ja < M) ? Pk[x + ja*n] : TF(0);
-                z.y = (jb < M) ? Pk[x + jb*n] : TF(0);
-                A[lpad(x)] = z;
-            }
         __syncthreads();
-        T* Z = fft_row<TF, ENG>(A, tws, tw, plan, -1, lane);
-        // Stage the two half-spectra packed in n slots: in the row buffer itself
-        // for the in-place engine (through registers), else in the free buffer.
-        int soff;
-        if (plan.fast)
+        T* Z = fft_row_pingpong<TF>(A, A + row_half(n), plan, tw, -1, lane);
+        // Stage the two half-spectra packed in n slots in the free buffer.
+        const int soff = (Z == A) ? row_half(n) : 0;
+        T* S = rows + row*re + soff;
+        for (int kx = lane; kx < nx; kx += 64)
         {
-            T xs[MAXQ][2];
-            #pragma unroll
-            for (int q = 0; q < MAXQ; ++q)
-            {
-                const int kx = lane + 64*q;
-                if (kx < nx) unpack_pair<TF>(Z[lpad(kx)], Z[lpad((n - kx) % n)], xs[q][0], xs[q][1]);
-            }
-            __syncthreads();
-            #pragma unroll
-            for (int q = 0; q < MAXQ; ++q)
-            {
-                const int kx = lane + 64*q;
-                if (kx < nx) stage_store<TF>(A, kx, n, xs[q][0], xs[q][1]);
-            }
-            soff = 0;
-        }
-        else
-        {
-            soff = (Z == A) ? row_half(n) : 0;
-            T* S = rows + row*re + soff;
-            for (int kx = lane; kx < nx; kx += 64)
-            {
-                T xa, xb;
-                unpack_pair<TF>(Z[lpad(kx)], Z[lpad((n - kx) % n)], xa, xb);
-                stage_store<TF>(S, kx, n, xa, xb);
-            }
+            T xa, xb;
+            unpack_pair<TF>(Z[lpad(kx)], Z[lpad((n - kx) % n)], xa, xb);
+            stage_store<TF>(S, kx, n, xa, xb);
         }
         __syncthreads();
         // The block writes C[k][kx][j0 .. j0+2RB) with consecutive threads on consecutive j.
-        const int nthr = 64*blockDim.y, tid = lane + 64*row;
+        const int nthr = 64*RB, tid = lane + 64*row;
         const int JB = 2*RB;
         T* Ck = C + static_cast<size_t>(k)*nx*M;
         for (int idx = tid; idx < nx*JB; idx += nthr)
@@ -243,7 +203,7 @@ namespace
         }
     }
 
-    template<typename TF, int ENG>
+    template<typename TF>
     struct fft_x_fwd_k
     {
         static constexpr int NT = 256, MINB = 0;
@@ -251,30 +211,28 @@ namespace
         Pin_args<TF> pin; int fuse_in;
         __device__ __forceinline__ void operator()(const Bid& bid_) const
         {
-            fft_x_fwd_g<TF, ENG>(P, C, plan, tw, RB, g, pmean, pin, fuse_in, bid_);
+            fft_x_fwd_g<TF>(P, C, plan, tw, RB, g, pmean, pin, fuse_in, bid_);
         }
     };
 
     // y transform (forward sign -1 or inverse +1) of RB contiguous rows of C;
     // the inverse divides by jtot as src/fft.cxx:420 does.
-    template<typename TF, int ENG>
+    template<typename TF>
     __device__ __forceinline__ void fft_y_g(cplx<TF>* __restrict__ C, const Plan& plan, const double2* __restrict__ tw,
                                             int sign, int nrows, int RB, const Bid& bid_)
     {
         using T = cplx<TF>;
         extern __shared__ unsigned char smem_raw[];
-        T* tws = reinterpret_cast<T*>(smem_raw);
         const int n = plan.n, re = row_elems(plan);
         const int row = threadIdx.y, lane = threadIdx.x;
         const int r = bid_.x*RB + row;
-        T* A = tws + tw_elems(plan) + row*re;
-        if (plan.fast) load_twiddles<TF>(tws, tw, n);
+        T* A = reinterpret_cast<T*>(smem_raw) + row*re;
         const bool active = r < nrows;
         T* Cr = C + static_cast<size_t>(active ? r : 0)*n;
         if (active)
             for (int x = lane; x < n; x += 64) A[lpad(x)] = Cr[x];
         __syncthreads();
-        T* Z = fft_row<TF, ENG>(A, tws, tw, plan, sign, lane);
+        T* Z = fft_row_pingpong<TF>(A, A + row_half(n), plan, tw, sign, lane);
         if (!active) return;
         if (sign < 0)
             for (int x = lane; x < n; x += 64) Cr[x] = Z[lpad(x)];
@@ -285,14 +243,14 @@ namespace
         }
     }
 
-    template<typename TF, int ENG>
+    template<typename TF>
     struct fft_y_k
     {
         static constexpr int NT = 256, MINB = 0;
         cplx<TF>* C; Plan plan; const double2* tw; int sign; int nrows; int RB;
         __device__ __forceinline__ void operator()(const Bid& bid_) const
         {
-            fft_y_g<TF, ENG>(C, plan, tw, sign, nrows, RB, bid_);
+            fft_y_g<TF>(C, plan, tw, sign, nrows, RB, bid_);
         }
     };
 
@@ -1250,62 +1208,45 @@ namespace
     // Inverse x transform and scatter into the ghosted p (Pres_2::solve tail,
     // src/pres_2.cxx:336-361): interior, the periodic halos of the rows the
     // block owns, and the bottom ghost level p[kstart-1] = p[kstart].
-    template<typename TF, int ENG>
+    template<typename TF>
     __device__ __forceinline__ void fft_x_bwd_g(const cplx<TF>* __restrict__ C, TF* __restrict__ p,
                                                 const Plan& plan, const double2* __restrict__ tw, int RB, Gd g, const Bid& bid_)
     {
         using T = cplx<TF>;
         extern __shared__ unsigned char smem_raw[];
-        T* tws = reinterpret_cast<T*>(smem_raw);
         const int n = plan.n, nx = n/2 + 1, M = g.jtot, re = row_elems(plan);
-        T* rows = tws + tw_elems(plan);
+        T* rows = reinterpret_cast<T*>(smem_raw);
         const int row = threadIdx.y, lane = threadIdx.x;
         const int k = bid_.y;
         const int j0 = bid_.x*2*RB;
-        const int nthr = 64*blockDim.y, tid = lane + 64*row;
+        const int nthr = 64*RB, tid = lane + 64*row;
         const int JB = 2*RB;
-        if (plan.fast) load_twiddles<TF>(tws, tw, n);
         const T* Ck = C + static_cast<size_t>(k)*nx*M;
-        // Stage the block's spectra packed as in the forward kernel; the DC and
-        // Nyquist entries of a real row are real.  The staging buffer is the row
-        // buffer itself (in-place engine) or the row's second buffer (fallback).
-        const int soff = plan.fast ? 0 : row_half(n);
-        // in chunks of SB loads per thread, all in flight before their LDS stores
-        constexpr int SB = 8;
-        for (int base = tid; base < nx*JB; base += SB*nthr)
+        // Stage the block's spectra packed as in the forward kernel, in the
+        // row's second buffer; the DC and Nyquist entries of a real row are real.
+        const int soff = row_half(n);
+        for (int idx = tid; idx < nx*JB; idx += nthr)
         {
-            T vals[SB];
-            #pragma unroll
-            for (int u = 0; u < SB; ++u)
+            const int kx = idx / JB, jl = idx % JB;
+            const int r = jl >> 1, part = jl & 1;
+            const int j = j0 + jl;
+            T val; val.x = TF(0); val.y = TF(0);
+            if (j < M) val = Ck[static_cast<size_t>(kx)*M + j];
+            T* Sr = rows + r*re + soff;
+            if (kx == 0 || 2*kx == n)
             {
-                const int idx = base + u*nthr;
-                const int j = j0 + idx % JB;
-                vals[u].x = TF(0); vals[u].y = TF(0);
-                if (idx < nx*JB && j < M) vals[u] = Ck[static_cast<size_t>(idx / JB)*M + j];
+                TF* d = reinterpret_cast<TF*>(&Sr[kx == 0 ? 0 : 1]);
+                d[part] = val.x;
             }
-            #pragma unroll
-            for (int u = 0; u < SB; ++u)
-            {
-                const int idx = base + u*nthr;
-                if (idx >= nx*JB) break;
-                const int kx = idx / JB, jl = idx % JB;
-                const int r = jl >> 1, part = jl & 1;
-                const T val = vals[u];
-                T* Sr = rows + r*re + soff;
-                if (kx == 0 || 2*kx == n)
-                {
-                    TF* d = reinterpret_cast<TF*>(&Sr[kx == 0 ? 0 : 1]);
-                    d[part] = val.x;
-                }
-                else
-                    Sr[lpad(stage_base(kx, n) + part)] = val;
-            }
+            else
+                Sr[lpad(stage_base(kx, n) + part)] = val;
         }
         __syncthreads();
         T* A = rows + row*re;
         const T* B = A + soff;
         // Hermitian extension of both spectra and packing Z = Xa + i Xb.
-        auto zval = [&](int x) -> T {
+        for (int x = lane; x < n; x += 64)
+        {
             T xa, xb;
             const int kx = (x <= n/2) ? x : n - x;
             if (kx == 0 || 2*kx == n)
@@ -1320,30 +1261,10 @@ namespace
                 if (x > n/2) { xa.y = -xa.y; xb.y = -xb.y; }
             }
             T z; z.x = xa.x - xb.y; z.y = xa.y + xb.x;
-            return z;
-        };
-        if (plan.fast)
-        {
-            constexpr int MAXX = 2*MAXQ;   // n/64 values per lane, n <= 1024
-            T zs[MAXX];
-            #pragma unroll
-            for (int q = 0; q < MAXX; ++q)
-            {
-                const int x = lane + 64*q;
-                if (x < n) zs[q] = zval(x);
-            }
-            __syncthreads();
-            #pragma unroll
-            for (int q = 0; q < MAXX; ++q)
-            {
-                const int x = lane + 64*q;
-                if (x < n) A[lpad(x)] = zs[q];
-            }
+            A[lpad(x)] = z;
         }
-        else
-            for (int x = lane; x < n; x += 64) A[lpad(x)] = zval(x);
         __syncthreads();
-        T* Z = fft_row<TF, ENG>(A, tws, tw, plan, +1, lane);
+        T* Z = fft_row_pingpong<TF>(A, A + soff, plan, tw, +1, lane);
         const int ja = j0 + 2*row, jb = ja + 1;
         const int jj = g.icells, kk = g.ijcells;
         const TF ni = TF(1)/TF(n);   // the /itot of src/fft.cxx:446, exact for powers of two
@@ -1374,14 +1295,14 @@ namespace
         }
     }
 
-    template<typename TF, int ENG>
+    template<typename TF>
     struct fft_x_bwd_k
     {
         static constexpr int NT = 256, MINB = 0;
         const cplx<TF>* C; TF* p; Plan plan; const double2* tw; int RB; Gd g;
         __device__ __forceinline__ void operator()(const Bid& bid_) const
         {
-            fft_x_bwd_g<TF, ENG>(C, p, plan, tw, RB, g, bid_);
+            fft_x_bwd_g<TF>(C, p, plan, tw, RB, g, bid_);
         }
     };
 
@@ -1651,19 +1572,15 @@ namespace
             red[1 + blockIdx.x + gridDim.x*(blockIdx.y + gridDim.y*blockIdx.z)] = sm[0];
     }
 
-    // Rows per block so that the twiddle table and the row buffers fit in 64 KiB.
+    // Rows per block so that the row buffers fit in 64 KiB.
     int rows_per_block(const Plan& p, size_t elem)
     {
-        const size_t budget = 65536 / elem;          // complex elements
-        const size_t per_row = static_cast<size_t>(row_elems(p));
-        const size_t tw = static_cast<size_t>(tw_elems(p));
-        const size_t avail = budget > tw ? budget - tw : 0;
-        return std::max(1, std::min(4, static_cast<int>(avail / per_row)));
+        return std::max(1, std::min(4, static_cast<int>(65536/elem/static_cast<size_t>(row_elems(p)))));
     }
 
     size_t lds_bytes(const Plan& p, int RB, size_t elem)
     {
-        return (static_cast<size_t>(tw_elems(p)) + static_cast<size_t>(RB)*row_elems(p))*elem;
+        return static_cast<size_t>(RB)*row_elems(p)*elem;
     }
 
     template<typename TF>
@@ -1768,22 +1685,8 @@ namespace
         t = Pres_tables<TF>();
     }
 
-    // Calls f with the plan's engine of the general kernels.  FP64 comes here
-    // only for lengths without a lane-group plan (1, 686, 882 and some above
-    // 1024), none of which the in-place engines take (1 has no pass).
-    template<typename TF, typename F>
-    void with_engine(const Plan& p, F f)
-    {
-        if constexpr (std::is_same<TF, float>::value)
-        {
-            if (p.engine == FFT_FAST) return f(std::integral_constant<int, FFT_FAST>{});
-            if (p.engine == FFT_FAST_WIDE) return f(std::integral_constant<int, FFT_FAST_WIDE>{});
-        }
-        f(std::integral_constant<int, FFT_PINGPONG>{});
-    }
-
     // y transform of nrows contiguous rows: the wave-per-row kernel for n = 128,
-    // 256 and 512, lane groups where there is a plan, the general engine
+    // 256 and 512, lane groups where there is a plan, the ping-pong engine
     // otherwise.
     template<typename TF, int R>
     void launch_fft_y_wave(mhh_ctx* c, cplx<TF>* C, const double* tw, int sign, int nrows)
@@ -1811,9 +1714,7 @@ namespace
                 const size_t ldsy = lds_bytes(py, RBy, sizeof(cplx<TF>));
                 const auto* t2 = reinterpret_cast<const double2*>(tw);
                 const dim3 grd((nrows + RBy - 1)/RBy), blk(64, RBy);
-                with_engine<TF>(py, [&](auto e) {
-                    launch(c, fft_y_k<TF, decltype(e)::value>{C, py, t2, sign, nrows, RBy}, grd, blk, ldsy);
-                });
+                launch(c, fft_y_k<TF>{C, py, t2, sign, nrows, RBy}, grd, blk, ldsy);
             }
         }
         return check_launch(name);
@@ -1926,8 +1827,8 @@ namespace
 
     // rk3 >= 0: apply the gradient together with the RK3 update of substep
     // rk3 (time step rkdt) instead of Pres_2::output alone.
-    // Forward x transform through the general engine (the right-hand side
-    // evaluated in the kernel when fuse_in, else read from P).
+    // Forward x transform of a length without a lane-group plan (the right-hand
+    // side evaluated in the kernel when fuse_in, else read from P).
     template<typename TF>
     int fft_x_fwd_general(mhh_ctx* c, const TF* P, cplx<TF>* C, const Plan& px, const Pres_tables<TF>& t,
                           const Pin_args<TF>& pin, int fuse_in)
@@ -1941,9 +1842,7 @@ namespace
           const auto* t2 = reinterpret_cast<const double2*>(t.twx);
           const double* pm = c->mixed ? c->pm_mean : nullptr;
           const dim3 blk(64, RB);
-          with_engine<TF>(px, [&](auto e) {
-              launch(c, fft_x_fwd_k<TF, decltype(e)::value>{P, C, px, t2, RB, g, pm, pin, fuse_in}, grd, blk, lds);
-          }); }
+          launch(c, fft_x_fwd_k<TF>{P, C, px, t2, RB, g, pm, pin, fuse_in}, grd, blk, lds); }
         return check_launch("fft_x_fwd");
     }
 
@@ -1977,11 +1876,10 @@ namespace
                         && g.igc <= 32;
         const bool xdft = !xwave && dft_applies(c, N);
         const bool xrow = !xwave && !xdft && c->row_px.n;
-        // The wave and lane-group x transforms evaluate the right-hand side
-        // themselves (and, in the mixed mode, the FP64 plane sums); the general
-        // engine does so except in the mixed mode, whose plane means come
-        // first, as they do for the matrix-core transform.
-        const int fuse_in = (xwave || xrow || !c->mixed) ? 1 : 0;
+        // The wave x transforms evaluate the right-hand side themselves (and, in
+        // the mixed mode, the FP64 plane sums); the others do so except in the
+        // mixed mode, whose plane means come first.
+        const int fuse_in = (xwave || !c->mixed) ? 1 : 0;
         const Pres_tables<double>& d = c->td;
         const size_t mm_lds = sizeof(double)*K;
         if (!fuse_in)
@@ -2004,26 +1902,24 @@ namespace
         const bool ywave = !c->fft_generic && !c->ytri_split && (M == 128 || M == 256 || M == 512);
         const int packed = xwave && ywave ? 1 : 0;
         // 2. forward x transform
-        if (xwave || xrow)
+        if (xwave)
         {
             const int mode = c->mixed ? 3 : 2;
-            if (xwave) MHH_CHECK(fft_x_fwd_wave<TF>(c, P, C, t.twx, mode, p, dxi, dyi, dti, "pres_in_fft_x", packed));
-            else MHH_CHECK((row_x_fwd<TF, T>(c, C, t.twx, c->mixed ? c->pm_part : nullptr, p, dxi, dyi, dti)));
+            MHH_CHECK(fft_x_fwd_wave<TF>(c, P, C, t.twx, mode, p, dxi, dyi, dti, "pres_in_fft_x", packed));
             if (c->mixed)
             {
-                const int nparts = xwave ? M/(2*xwaves<TF>()) : row_x_nparts(c);
-                { mhh::Timer _t(c, "pres_mean"); launch(c, mean_mode_k{c->pm_part, nparts, c->pm_mean,
+                { mhh::Timer _t(c, "pres_mean"); launch(c, mean_mode_k{c->pm_part, M/(2*xwaves<TF>()), c->pm_mean,
                         c->pbar, c->dpbar, d.a, d.dz2, c->pm_coef, 1./(double(N)*double(M)), g}, 1, 256, mm_lds); }
                 MHH_CHECK(check_launch("mean_mode"));
             }
         }
-        else if constexpr (std::is_same<TF, float>::value)
-        {
-            if (xdft) MHH_CHECK(dft_x_fwd(c, P, C, c->pm_mean));
-            else MHH_CHECK(fft_x_fwd_general<TF>(c, P, C, px, t, pin, fuse_in));
-        }
         else
-            MHH_CHECK(fft_x_fwd_general<TF>(c, P, C, px, t, pin, fuse_in));
+        {
+            if constexpr (std::is_same<TF, float>::value)
+                if (xdft) MHH_CHECK(dft_x_fwd(c, P, C, c->pm_mean));
+            if (xrow) MHH_CHECK((row_x_fwd<TF, T>(c, fuse_in ? nullptr : P, C, t.twx, p, dxi, dyi, dti)));
+            else if (!xdft) MHH_CHECK(fft_x_fwd_general<TF>(c, P, C, px, t, pin, fuse_in));
+        }
         const int nrows = nx*K;
         if (ywave)
         {
@@ -2083,9 +1979,7 @@ namespace
                 const auto* t2 = reinterpret_cast<const double2*>(t.twx);
                 mhh::Timer _t(c, "fft_x_bwd");
                 const dim3 blk(64, RB);
-                with_engine<TF>(px, [&](auto e) {
-                    launch(c, fft_x_bwd_k<TF, decltype(e)::value>{C, P, px, t2, RB, g}, grd, blk, lds);
-                });
+                launch(c, fft_x_bwd_k<TF>{C, P, px, t2, RB, g}, grd, blk, lds);
                 MHH_CHECK(check_launch("fft_x_bwd"));
             }
         }
@@ -2227,9 +2121,8 @@ namespace mhh
         {
             const size_t K = c->gd.ktot, nk = c->gd.kcells;
             // partial plane sums: PM_CHUNKS per level (plane_sum_g) or one per
-            // block of rows (the wave and lane-group x transforms)
-            const size_t nparts = std::max<size_t>({PM_CHUNKS, static_cast<size_t>(c->gd.jtot + 7)/8,
-                                                    static_cast<size_t>(row_x_nparts(c))});
+            // block of 8 rows (the wave x transform)
+            const size_t nparts = std::max<size_t>(PM_CHUNKS, (c->gd.jtot + 7)/8);
             MHH_CHECK(check_hip(hipMalloc(&c->pm_part, sizeof(double)*K*nparts), "hipMalloc(pm_part)"));
             MHH_CHECK(check_hip(hipMalloc(&c->pm_mean, sizeof(double)*K), "hipMalloc(pm_mean)"));
             MHH_CHECK(check_hip(hipMalloc(&c->pbar, sizeof(double)*nk), "hipMalloc(pbar)"));

@@ -1,6 +1,6 @@
 // mhh_rowfft.hip -- the x and y transforms of the pressure projection for
 // every length that has no kernel of its own (mhh_rowfft.h: lane groups,
-// two to four passes): the forward x transform with the right-hand side of
+// a few passes): the forward x transform with the right-hand side of
 // Pres_2::input (src/pres_2.cxx:155-196) evaluated into its first pass, the y
 // transforms in place on the spectrum's rows, and the inverse x transform into
 // the ghosted p.  They replace FFTW's R2HC/HC2R and their per-slice order
@@ -8,20 +8,13 @@
 //
 // What bounds them: the memory traffic of one pass over the fields (x, forward)
 // or the spectrum, and on small grids the latency of the passes.  Measured, against
-// the general engine of mhh_fft.h (radices up to 8 and 5, block barriers between
-// passes) that they replace in FP64 and the mixed mode:
-//   768 x 384 x 256 FP64: forward x 943 us (7 passes over the fields, 4.5 TB/s;
-//     1629), y 267 (4.5 TB/s; 416), inverse x 356 (764)
-//   240 x 180 x 120 FP64: 95, 26.6, 36.6 us (102, 41.5, 55.9)
-//   90 x 75 x 60 FP64: 13.8, 7.8, 9.1 us (15.9, 8.9, 13.1)
-// and lengths the general engine had only its ping-pong fallback for, e.g. 960 x
-// 500 x 58 FP64 and its like: projection and step about 2 times as fast.  In the
-// mixed mode the right-hand side, its plane sums and the transform are one kernel
-// (192 x 96 x 64: 13.9 us for 26.3).  Plain FP32 keeps the general engine: its
-// projection carries the horizontal mean through FP32 transforms and sweeps, and
-// rows in another order change the velocities of a 96 x 96 x 64 model by 4e-3
-// after two steps, about the error it has against FP64; what its callers get
-// stays what it was.
+// the block-wide engine (a wave per row, block barriers between passes) that they
+// replace, bit for bit:
+//   768 x 384 x 256 FP64: forward x 956 us (7 passes over the fields, 4.5 TB/s;
+//     1629), y 382 (416), inverse x 384 (764)
+//   90 x 75 x 60 FP64: 14.3, 7.9, 8.9 us (15.9, 8.9, 13.1)
+// and where that engine had only its ping-pong fallback (mhh_fft.h): the projection
+// of 960 x 500 x 58 FP64 1.36 ms instead of 5.00.
 #include <algorithm>
 
 #include "mhh_batch.h"
@@ -103,14 +96,12 @@ namespace
     }
 
     // Forward x transform of the pairs of real rows (j, j+1) of level k packed
-    // as a + i b; writes C[k][kx][j] for kx <= itot/2.  FP32 rows go in minus
-    // their FP64 mean and bin 0 is set to the FP64 sum afterwards: only bin 0
-    // changes, and the other bins round against the fluctuations instead of the
-    // mean.  part (mixed mode): the block's FP64 sum of the right-hand side,
-    // part[k*nbj + bj], whose mode the FP64 path solves.
-    template<typename TF, int VALS>
+    // as a + i b; writes C[k][kx][j] for kx <= itot/2.  The rows are the right-hand
+    // side evaluated here or (P, mixed mode) read from the dense array P minus the
+    // plane mean pmean[k], whose mode the FP64 path solves.
+    template<typename TF, int VALS, int ARITH>
     __device__ __forceinline__ void row_x_fwd_g(cplx<TF>* __restrict__ C, const Row_plan& p, const double2* __restrict__ tw,
-                                                double* __restrict__ part,
+                                                const TF* __restrict__ P, const double* __restrict__ pmean,
                                                 const TF* __restrict__ u, const TF* __restrict__ v, const TF* __restrict__ w,
                                                 const TF* __restrict__ ut, const TF* __restrict__ vt, const TF* __restrict__ wt,
                                                 const TF* __restrict__ dzi, const TF* __restrict__ rho,
@@ -118,9 +109,7 @@ namespace
                                                 const Bid& bid_)
     {
         using T = cplx<TF>;
-        constexpr bool SUM = sizeof(TF) == 4;
         extern __shared__ unsigned char smem_raw[];
-        __shared__ double rsum[SUM ? 64 : 1];
         T* tws = reinterpret_cast<T*>(smem_raw);
         const int n = p.n, nx = n/2 + 1, M = g.jtot, stride = row_stride(n);
         T* rows = tws + lpad(n - 1) + 1;
@@ -140,43 +129,38 @@ namespace
         const Row_rhs<TF> rhs{u, v, w, ut, vt, wt, rho[kc], rhoh[kc], rhoh[kc+1], dzi[kc], dxi, dyi, dti, n, g.ijcells,
                         base + jra*g.icells, base + jrb*g.icells, base + (jra + 1)*g.icells, base + (jrb + 1)*g.icells,
                         base + (jra + 1 == M ? 0 : jra + 1)*g.icells, base + (jrb + 1 == M ? 0 : jrb + 1)*g.icells};
-        double sx = 0., sy = 0.;
         // a lane's elements in steps of four, their loads in flight together
         constexpr int RU = 4;
+        const bool dense = sizeof(TF) == 4 && P;
+        const double m = dense ? pmean[k] : 0.;
+        const TF* __restrict__ Pa = P + (static_cast<size_t>(k)*M + jra)*n;
+        const TF* __restrict__ Pb = P + (static_cast<size_t>(k)*M + jrb)*n;
         for (int x0 = l; x0 < n; x0 += RU*L)
         {
             T z[RU];
-            #pragma unroll
-            for (int q = 0; q < RU; ++q) z[q] = rhs(min(x0 + q*L, n - 1));
+            if (dense)
+            {
+                #pragma unroll
+                for (int q = 0; q < RU; ++q)
+                {
+                    const int x = min(x0 + q*L, n - 1);
+                    z[q].x = Pa[x]; z[q].y = Pb[x];
+                }
+                #pragma unroll
+                for (int q = 0; q < RU; ++q) { z[q].x = TF(double(z[q].x) - m); z[q].y = TF(double(z[q].y) - m); }
+            }
+            else
+            {
+                #pragma unroll
+                for (int q = 0; q < RU; ++q) z[q] = rhs(min(x0 + q*L, n - 1));
+            }
             #pragma unroll
             for (int q = 0; q < RU; ++q)
-                if (x0 + q*L < n)
-                {
-                    row[lpad(x0 + q*L)] = z[q];
-                    if (SUM) { sx += double(z[q].x); sy += double(z[q].y); }
-                }
-        }
-        if (SUM)
-        {
-            for (int o = L >> 1; o > 0; o >>= 1) { sx += __shfl_xor(sx, o); sy += __shfl_xor(sy, o); }
-            const TF mx = TF(sx/n), my = TF(sy/n);
-            for (int x = l; x < n; x += L) { T z = row[lpad(x)]; z.x -= mx; z.y -= my; row[lpad(x)] = z; }
+                if (x0 + q*L < n) row[lpad(x0 + q*L)] = z[q];
         }
         __syncthreads();   // the roots
-        row_fft<TF, VALS>(row, tws, p, l);
-        if (SUM && l == 0)
-        {
-            T z; z.x = TF(sx); z.y = TF(sy);
-            row[0] = z;
-            rsum[rl] = (ja < M ? sx : 0.) + (ja + 1 < M ? sy : 0.);
-        }
+        row_fft<TF, VALS, ARITH, ROW_X_FWD>(row, tws, p, l);
         __syncthreads();
-        if (SUM && part && tid == 0)
-        {
-            double s = 0.;
-            for (int r = 0; r < RP; ++r) s += rsum[r];
-            part[static_cast<size_t>(k)*xg.nbj + bj] = s;
-        }
         // The half-spectra of the rows a, b from Z = FFT(a + i b): Xa =
         // (Z[k] + conj Z[-k])/2, Xb = (Z[k] - conj Z[-k])/(2i), into C[k][kx][j],
         // consecutive threads on consecutive pairs
@@ -196,39 +180,40 @@ namespace
         }
     }
 
-    template<typename TF, int VALS>
+    template<typename TF, int VALS, int ARITH>
     struct row_x_fwd_k
     {
         static constexpr int NT = 64*xw<TF>(), MINB = 0;
-        cplx<TF>* C; Row_plan p; const double2* tw; double* part; const TF* u; const TF* v; const TF* w; const TF* ut;
+        cplx<TF>* C; Row_plan p; const double2* tw; const TF* P; const double* pmean; const TF* u; const TF* v; const TF* w; const TF* ut;
         const TF* vt; const TF* wt; const TF* dzi; const TF* rho; const TF* rhoh; TF dxi; TF dyi; TF dti; int nw; Xgrid xg;
         Gd g;
         __device__ __forceinline__ void operator()(const Bid& bid_) const
         {
-            row_x_fwd_g<TF, VALS>(C, p, tw, part, u, v, w, ut, vt, wt, dzi, rho, rhoh, dxi, dyi, dti, nw, xg, g, bid_);
+            row_x_fwd_g<TF, VALS, ARITH>(C, p, tw, P, pmean, u, v, w, ut, vt, wt, dzi, rho, rhoh, dxi, dyi, dti, nw, xg, g,
+                                         bid_);
         }
     };
 
     // The same outside a batch, with the pointers as __restrict__ kernel
     // parameters: the right-hand side's loads of a lane are then issued together.
-    template<typename TF, int VALS>
+    template<typename TF, int VALS, int ARITH>
     __global__ void __launch_bounds__(64*xw<TF>()) row_x_fwd_direct(
-            cplx<TF>* __restrict__ C, Row_plan p, const double2* __restrict__ tw, double* __restrict__ part,
+            cplx<TF>* __restrict__ C, Row_plan p, const double2* __restrict__ tw, const TF* __restrict__ P,
+            const double* __restrict__ pmean,
             const TF* __restrict__ u, const TF* __restrict__ v, const TF* __restrict__ w,
             const TF* __restrict__ ut, const TF* __restrict__ vt, const TF* __restrict__ wt,
             const TF* __restrict__ dzi, const TF* __restrict__ rho, const TF* __restrict__ rhoh,
             TF dxi, TF dyi, TF dti, int nw, Xgrid xg, Gd g)
     {
-        row_x_fwd_g<TF, VALS>(C, p, tw, part, u, v, w, ut, vt, wt, dzi, rho, rhoh, dxi, dyi, dti, nw, xg, g,
+        row_x_fwd_g<TF, VALS, ARITH>(C, p, tw, P, pmean, u, v, w, ut, vt, wt, dzi, rho, rhoh, dxi, dyi, dti, nw, xg, g,
                               Bid{static_cast<int>(blockIdx.x), 0, 0, static_cast<int>(gridDim.x), 1, 1});
     }
 
     // y transform of nrows contiguous rows of C in place, a lane group per row;
-    // waves walk the rows with a stride.  inv divides by jtot (src/fft.cxx:420).
-    // FP32 forward: the row minus its FP64 mean, bin 0 from the FP64 sum.
-    template<typename TF, int VALS>
+    // waves walk the rows with a stride.  INV divides by jtot (src/fft.cxx:420).
+    template<typename TF, int VALS, int ARITH, bool INV>
     __device__ __forceinline__ void row_y_g(cplx<TF>* __restrict__ C, const Row_plan& p, const double2* __restrict__ tw,
-                                            int nrows, int inv, int nw, const Bid& bid_)
+                                            int nrows, int nw, const Bid& bid_)
     {
         using T = cplx<TF>;
         extern __shared__ unsigned char smem_raw[];
@@ -245,8 +230,6 @@ namespace
             const int r = r0 + sub;
             const bool active = r < nrows;
             T* __restrict__ Cr = C + static_cast<size_t>(min(r, nrows - 1))*n;
-            double sx = 0., sy = 0.;
-            const bool sum = sizeof(TF) == 4 && !inv;
             constexpr int YU = 8;    // loads of a lane in flight
             for (int x0 = l; x0 < n; x0 += YU*L)
             {
@@ -255,44 +238,36 @@ namespace
                 for (int q = 0; q < YU; ++q) z[q] = Cr[min(x0 + q*L, n - 1)];
                 #pragma unroll
                 for (int q = 0; q < YU; ++q)
-                    if (x0 + q*L < n)
-                    {
-                        if (sum) { sx += double(z[q].x); sy += double(z[q].y); }
-                        row[lpad(x0 + q*L)] = inv ? T{z[q].y, z[q].x} : z[q];
-                    }
+                    if (x0 + q*L < n) row[lpad(x0 + q*L)] = z[q];
             }
-            if (sum)
-            {
-                for (int o = L >> 1; o > 0; o >>= 1) { sx += __shfl_xor(sx, o); sy += __shfl_xor(sy, o); }
-                const TF mx = TF(sx/n), my = TF(sy/n);
-                for (int x = l; x < n; x += L) { T z = row[lpad(x)]; z.x -= mx; z.y -= my; row[lpad(x)] = z; }
-            }
-            row_fft<TF, VALS>(row, tws, p, l);
-            if (sum && l == 0) row[0] = T{TF(sx), TF(sy)};
-            wave_lds_sync();
+            row_fft<TF, VALS, ARITH, INV ? ROW_Y_INV : ROW_Y_FWD>(row, tws, p, l);
             if (active)
                 for (int x = l; x < n; x += L)
                 {
-                    const T o = row[lpad(x)];
-                    Cr[x] = inv ? T{o.y*ni, o.x*ni} : o;
+                    T o = row[lpad(x)];
+                    if (INV) { o.x *= ni; o.y *= ni; }
+                    Cr[x] = o;
                 }
             wave_lds_sync();
         }
     }
 
-    template<typename TF, int VALS>
+    template<typename TF, int VALS, int ARITH, bool INV>
     struct row_y_k
     {
         static constexpr int NT = 256, MINB = 0;
-        cplx<TF>* C; Row_plan p; const double2* tw; int nrows; int inv; int nw;
-        __device__ __forceinline__ void operator()(const Bid& bid_) const { row_y_g<TF, VALS>(C, p, tw, nrows, inv, nw, bid_); }
+        cplx<TF>* C; Row_plan p; const double2* tw; int nrows; int nw;
+        __device__ __forceinline__ void operator()(const Bid& bid_) const
+        {
+            row_y_g<TF, VALS, ARITH, INV>(C, p, tw, nrows, nw, bid_);
+        }
     };
 
     // Inverse x transform (divides by itot, src/fft.cxx:446) of the row pairs of
     // C[k][kx][j] into the ghosted p: interior rows, their periodic images in the
     // y halo, the x halo columns and, at the lowest level, the ghost level
     // below (Pres_2::solve tail, src/pres_2.cxx:336-361).
-    template<typename TF, int VALS>
+    template<typename TF, int VALS, int ARITH>
     __device__ __forceinline__ void row_x_bwd_g(const cplx<TF>* __restrict__ C, TF* __restrict__ pf, const Row_plan& p,
                                                 const double2* __restrict__ tw, int nw, Xgrid xg, Gd g, const Bid& bid_)
     {
@@ -309,7 +284,7 @@ namespace
         const int RP = nw*rpw, psh = 31 - __clz(RP);
         const int j0 = bj*2*RP;
         // The packed spectrum Z = Xa + i Xb of a pair over all n bins from its two
-        // half-spectra (Hermitian), parts swapped for the inverse; consecutive
+        // half-spectra (Hermitian); consecutive
         // threads on consecutive pairs, several loads of a thread in flight
         const T* Ck = C + static_cast<size_t>(k)*nx*M;
         constexpr int SB = 4;
@@ -334,11 +309,11 @@ namespace
                     T* Sr = rows + (idx & (RP - 1))*stride;
                     T xa = va[q], xb = vb[q];
                     if (kx == 0 || 2*kx == n) { xa.y = TF(0); xb.y = TF(0); }   // real bins of a real row
-                    T z; z.x = xa.y + xb.x; z.y = xa.x - xb.y;
+                    T z; z.x = xa.x - xb.y; z.y = xa.y + xb.x;
                     Sr[lpad(kx)] = z;
                     if (kx > 0 && 2*kx < n)
                     {
-                        z.x = xb.x - xa.y; z.y = xa.x + xb.y;
+                        z.x = xa.x + xb.y; z.y = xb.x - xa.y;
                         Sr[lpad(n - kx)] = z;
                     }
                 }
@@ -347,7 +322,7 @@ namespace
         load_roots<TF>(tws, tw, n, tid, nthr);
         __syncthreads();
         T* row = rows + rl*stride;
-        row_fft<TF, VALS>(row, tws, p, l);
+        row_fft<TF, VALS, ARITH, ROW_X_INV>(row, tws, p, l);
         const TF ni = TF(1)/TF(n);   // exact for powers of two
         TF* __restrict__ pk = pf + static_cast<size_t>(k + g.kgc)*g.ijcells;
         for (int h = 0; h < 2; ++h)
@@ -365,7 +340,7 @@ namespace
                 int xi = x - g.igc;
                 xi = xi < 0 ? xi + n : xi >= n ? xi - n : xi;
                 const T z = row[lpad(xi)];
-                const TF val = (h ? z.x : z.y)*ni;
+                const TF val = (h ? z.y : z.x)*ni;
                 for (int e = 0; e < nd; ++e)
                 {
                     TF* __restrict__ pr = pk + x + static_cast<size_t>(dst[e])*g.icells;
@@ -376,16 +351,28 @@ namespace
         }
     }
 
-    template<typename TF, int VALS>
+    template<typename TF, int VALS, int ARITH>
     struct row_x_bwd_k
     {
         static constexpr int NT = 64*xw<TF>(), MINB = 0;
         const cplx<TF>* C; TF* pf; Row_plan p; const double2* tw; int nw; Xgrid xg; Gd g;
         __device__ __forceinline__ void operator()(const Bid& bid_) const
         {
-            row_x_bwd_g<TF, VALS>(C, pf, p, tw, nw, xg, g, bid_);
+            row_x_bwd_g<TF, VALS, ARITH>(C, pf, p, tw, nw, xg, g, bid_);
         }
     };
+
+    // Calls f with the plan's instance, (values per lane, arithmetic).
+    template<typename TF, typename F>
+    void with_instance(const Row_plan& p, F f)
+    {
+        auto arith = [&](auto v) {
+            if (p.arith == ROW_DIRECT) return f(v, std::integral_constant<int, ROW_DIRECT>{});
+            f(v, std::integral_constant<int, ROW_RADIX8>{});
+        };
+        if (p.vals == ROW_VALS) arith(std::integral_constant<int, ROW_VALS>{});
+        else arith(std::integral_constant<int, ROW_VALS_WIDE>{});
+    }
 
     template<typename TF>
     size_t row_lds(const Row_plan& p, int nw)
@@ -410,22 +397,12 @@ namespace mhh
     void row_plans_init(mhh_ctx* c)
     {
         const Gd& g = c->gd;
-        if (c->precision == MHH_FP32 && !c->mixed) return;
         make_row_plan(g.itot, static_cast<long long>(g.jtot + 1)/2*g.ktot, c->row_px);
         make_row_plan(g.jtot, static_cast<long long>(g.itot/2 + 1)*g.ktot, c->row_py);
     }
 
-    // Blocks per level of the forward x transform in the mixed mode.
-    int row_x_nparts(const mhh_ctx* c)
-    {
-        const Row_plan& p = c->row_px;
-        if (!p.n) return 0;
-        const int per = 2*row_waves<float>(p, xw<float>(), (c->gd.jtot + 1)/2)*(64 >> p.lsh);
-        return (c->gd.jtot + per - 1)/per;
-    }
-
     template<typename TF, typename T>
-    int row_x_fwd(mhh_ctx* c, T* C, const double* tw, double* part, const Prof<TF>& pr, TF dxi, TF dyi, TF dti)
+    int row_x_fwd(mhh_ctx* c, const TF* P, T* C, const double* tw, const Prof<TF>& pr, TF dxi, TF dyi, TF dti)
     {
         const Gd& g = c->gd;
         const Row_plan& p = c->row_px;
@@ -437,16 +414,18 @@ namespace mhh
         const TF* w = static_cast<const TF*>(c->f.w); const TF* ut = static_cast<const TF*>(c->f.ut);
         const TF* vt = static_cast<const TF*>(c->f.vt); const TF* wt = static_cast<const TF*>(c->f.wt);
         {
-            mhh::Timer _t(c, "pres_in_fft_x");
-#define MHH_RX(V) do { if (c->rec) launch(c, row_x_fwd_k<TF, V>{C, p, t2, part, u, v, w, ut, vt, wt, pr.dzi, pr.rhoref, \
-                pr.rhorefh, dxi, dyi, dti, nw, xg, g}, xg.nb, 64*nw, lds); \
-            else row_x_fwd_direct<TF, V><<<xg.nb, 64*nw, lds, c->stream>>>(C, p, t2, part, u, v, w, ut, vt, wt, pr.dzi, \
-                pr.rhoref, pr.rhorefh, dxi, dyi, dti, nw, xg, g); } while (0)
-            if (p.vals == ROW_VALS) MHH_RX(ROW_VALS);
-            else MHH_RX(ROW_VALS_WIDE);
-#undef MHH_RX
+            mhh::Timer _t(c, P ? "fft_x_fwd" : "pres_in_fft_x");
+            with_instance<TF>(p, [&](auto vc, auto ac) {
+                constexpr int V = decltype(vc)::value, A = decltype(ac)::value;
+                if (c->rec)
+                    launch(c, row_x_fwd_k<TF, V, A>{C, p, t2, P, c->pm_mean, u, v, w, ut, vt, wt, pr.dzi, pr.rhoref,
+                                                    pr.rhorefh, dxi, dyi, dti, nw, xg, g}, xg.nb, 64*nw, lds);
+                else
+                    row_x_fwd_direct<TF, V, A><<<xg.nb, 64*nw, lds, c->stream>>>(C, p, t2, P, c->pm_mean, u, v, w, ut, vt, wt,
+                        pr.dzi, pr.rhoref, pr.rhorefh, dxi, dyi, dti, nw, xg, g);
+            });
         }
-        return check_launch("pres_in_fft_x");
+        return check_launch(P ? "fft_x_fwd" : "pres_in_fft_x");
     }
 
     template<typename TF, typename T>
@@ -460,9 +439,11 @@ namespace mhh
         const auto* t2 = reinterpret_cast<const double2*>(tw);
         {
             mhh::Timer _t(c, name);
-            const int inv = sign > 0;
-            if (p.vals == ROW_VALS) launch(c, row_y_k<TF, ROW_VALS>{C, p, t2, nrows, inv, nw}, nb, 64*nw, lds);
-            else launch(c, row_y_k<TF, ROW_VALS_WIDE>{C, p, t2, nrows, inv, nw}, nb, 64*nw, lds);
+            with_instance<TF>(p, [&](auto vc, auto ac) {
+                constexpr int V = decltype(vc)::value, A = decltype(ac)::value;
+                if (sign < 0) launch(c, row_y_k<TF, V, A, false>{C, p, t2, nrows, nw}, nb, 64*nw, lds);
+                else launch(c, row_y_k<TF, V, A, true>{C, p, t2, nrows, nw}, nb, 64*nw, lds);
+            });
         }
         return check_launch(name);
     }
@@ -478,15 +459,18 @@ namespace mhh
         const auto* t2 = reinterpret_cast<const double2*>(tw);
         {
             mhh::Timer _t(c, "fft_x_bwd");
-            if (p.vals == ROW_VALS) launch(c, row_x_bwd_k<TF, ROW_VALS>{C, pf, p, t2, nw, xg, g}, xg.nb, 64*nw, lds);
-            else launch(c, row_x_bwd_k<TF, ROW_VALS_WIDE>{C, pf, p, t2, nw, xg, g}, xg.nb, 64*nw, lds);
+            with_instance<TF>(p, [&](auto vc, auto ac) {
+                launch(c, row_x_bwd_k<TF, decltype(vc)::value, decltype(ac)::value>{C, pf, p, t2, nw, xg, g}, xg.nb, 64*nw,
+                       lds);
+            });
         }
         return check_launch("fft_x_bwd");
     }
 
-    template int row_x_fwd<float, float2>(mhh_ctx*, float2*, const double*, double*, const Prof<float>&, float, float, float);
-    template int row_x_fwd<double, double2>(mhh_ctx*, double2*, const double*, double*, const Prof<double>&, double, double,
-                                   double);
+    template int row_x_fwd<float, float2>(mhh_ctx*, const float*, float2*, const double*, const Prof<float>&, float, float,
+                                              float);
+    template int row_x_fwd<double, double2>(mhh_ctx*, const double*, double2*, const double*, const Prof<double>&, double,
+                                                double, double);
     template int row_y<float, float2>(mhh_ctx*, float2*, const double*, int, int, const char*);
     template int row_y<double, double2>(mhh_ctx*, double2*, const double*, int, int, const char*);
     template int row_x_bwd<float, float2>(mhh_ctx*, const float2*, float*, const double*);
