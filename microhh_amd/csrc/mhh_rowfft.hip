@@ -98,8 +98,11 @@ namespace
     // Forward x transform of the pairs of real rows (j, j+1) of level k packed
     // as a + i b; writes C[k][kx][j] for kx <= itot/2.  The rows are the right-hand
     // side evaluated here or (P, mixed mode) read from the dense array P minus the
-    // plane mean pmean[k], whose mode the FP64 path solves.
-    template<typename TF, int VALS, int ARITH>
+    // plane mean pmean[k], whose mode the FP64 path solves (DENSE, a kernel of
+    // its own: chosen at run time, it kept the right-hand side's loads from being
+    // issued together, and the projection of 360 x 250 x 100 FP32 took 343 us
+    // instead of 286).
+    template<typename TF, int VALS, int ARITH, bool DENSE>
     __device__ __forceinline__ void row_x_fwd_g(cplx<TF>* __restrict__ C, const Row_plan& p, const double2* __restrict__ tw,
                                                 const TF* __restrict__ P, const double* __restrict__ pmean,
                                                 const TF* __restrict__ u, const TF* __restrict__ v, const TF* __restrict__ w,
@@ -131,14 +134,13 @@ namespace
                         base + (jra + 1 == M ? 0 : jra + 1)*g.icells, base + (jrb + 1 == M ? 0 : jrb + 1)*g.icells};
         // a lane's elements in steps of four, their loads in flight together
         constexpr int RU = 4;
-        const bool dense = sizeof(TF) == 4 && P;
-        const double m = dense ? pmean[k] : 0.;
+        const double m = DENSE ? pmean[k] : 0.;
         const TF* __restrict__ Pa = P + (static_cast<size_t>(k)*M + jra)*n;
         const TF* __restrict__ Pb = P + (static_cast<size_t>(k)*M + jrb)*n;
         for (int x0 = l; x0 < n; x0 += RU*L)
         {
             T z[RU];
-            if (dense)
+            if constexpr (DENSE)
             {
                 #pragma unroll
                 for (int q = 0; q < RU; ++q)
@@ -180,7 +182,7 @@ namespace
         }
     }
 
-    template<typename TF, int VALS, int ARITH>
+    template<typename TF, int VALS, int ARITH, bool DENSE>
     struct row_x_fwd_k
     {
         static constexpr int NT = 64*xw<TF>(), MINB = 0;
@@ -189,14 +191,14 @@ namespace
         Gd g;
         __device__ __forceinline__ void operator()(const Bid& bid_) const
         {
-            row_x_fwd_g<TF, VALS, ARITH>(C, p, tw, P, pmean, u, v, w, ut, vt, wt, dzi, rho, rhoh, dxi, dyi, dti, nw, xg, g,
+            row_x_fwd_g<TF, VALS, ARITH, DENSE>(C, p, tw, P, pmean, u, v, w, ut, vt, wt, dzi, rho, rhoh, dxi, dyi, dti, nw, xg, g,
                                          bid_);
         }
     };
 
     // The same outside a batch, with the pointers as __restrict__ kernel
     // parameters: the right-hand side's loads of a lane are then issued together.
-    template<typename TF, int VALS, int ARITH>
+    template<typename TF, int VALS, int ARITH, bool DENSE>
     __global__ void __launch_bounds__(64*xw<TF>()) row_x_fwd_direct(
             cplx<TF>* __restrict__ C, Row_plan p, const double2* __restrict__ tw, const TF* __restrict__ P,
             const double* __restrict__ pmean,
@@ -205,7 +207,7 @@ namespace
             const TF* __restrict__ dzi, const TF* __restrict__ rho, const TF* __restrict__ rhoh,
             TF dxi, TF dyi, TF dti, int nw, Xgrid xg, Gd g)
     {
-        row_x_fwd_g<TF, VALS, ARITH>(C, p, tw, P, pmean, u, v, w, ut, vt, wt, dzi, rho, rhoh, dxi, dyi, dti, nw, xg, g,
+        row_x_fwd_g<TF, VALS, ARITH, DENSE>(C, p, tw, P, pmean, u, v, w, ut, vt, wt, dzi, rho, rhoh, dxi, dyi, dti, nw, xg, g,
                               Bid{static_cast<int>(blockIdx.x), 0, 0, static_cast<int>(gridDim.x), 1, 1});
     }
 
@@ -417,12 +419,18 @@ namespace mhh
             mhh::Timer _t(c, P ? "fft_x_fwd" : "pres_in_fft_x");
             with_instance<TF>(p, [&](auto vc, auto ac) {
                 constexpr int V = decltype(vc)::value, A = decltype(ac)::value;
-                if (c->rec)
-                    launch(c, row_x_fwd_k<TF, V, A>{C, p, t2, P, c->pm_mean, u, v, w, ut, vt, wt, pr.dzi, pr.rhoref,
-                                                    pr.rhorefh, dxi, dyi, dti, nw, xg, g}, xg.nb, 64*nw, lds);
-                else
-                    row_x_fwd_direct<TF, V, A><<<xg.nb, 64*nw, lds, c->stream>>>(C, p, t2, P, c->pm_mean, u, v, w, ut, vt, wt,
-                        pr.dzi, pr.rhoref, pr.rhorefh, dxi, dyi, dti, nw, xg, g);
+                auto go = [&](auto dc) {
+                    constexpr bool D = decltype(dc)::value;
+                    if (c->rec)
+                        launch(c, row_x_fwd_k<TF, V, A, D>{C, p, t2, P, c->pm_mean, u, v, w, ut, vt, wt, pr.dzi, pr.rhoref,
+                                                           pr.rhorefh, dxi, dyi, dti, nw, xg, g}, xg.nb, 64*nw, lds);
+                    else
+                        row_x_fwd_direct<TF, V, A, D><<<xg.nb, 64*nw, lds, c->stream>>>(C, p, t2, P, c->pm_mean, u, v, w, ut,
+                            vt, wt, pr.dzi, pr.rhoref, pr.rhorefh, dxi, dyi, dti, nw, xg, g);
+                };
+                if constexpr (sizeof(TF) == 4)
+                    if (P) return go(std::true_type{});
+                go(std::false_type{});
             });
         }
         return check_launch(P ? "fft_x_fwd" : "pres_in_fft_x");
