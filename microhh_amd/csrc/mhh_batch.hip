@@ -8,7 +8,7 @@
 // runs them merged: the members whose next kernel is of the same type run it
 // in one launch, whose blocks a table of first blocks deals to the members.
 // Members of different sizes take different transform kernels (the wave
-// kernels for 128, 256, 512 points, the general engine otherwise); the merge
+// kernels for 128, 256, 512 points, lane groups otherwise); the merge
 // then issues each kernel type once over the members that use it.
 #include <algorithm>
 #include <cstring>
