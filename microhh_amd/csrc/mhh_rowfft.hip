@@ -127,8 +127,10 @@ namespace
         T* row = rows + rl*stride;
 
         const int kc = k + g.kgc, base = g.igc + g.jgc*g.icells + kc*g.ijcells;
-        // rows past the last are computed on the last (in bounds) and not stored
+        // rows past the last are read as the last (in bounds) and not stored; an
+        // odd last row is packed with zero, so that it is rounded by itself
         const int jra = min(ja, M - 1), jrb = min(ja + 1, M - 1);
+        const bool pair = ja + 1 < M;
         const Row_rhs<TF> rhs{u, v, w, ut, vt, wt, rho[kc], rhoh[kc], rhoh[kc+1], dzi[kc], dxi, dyi, dti, n, g.ijcells,
                         base + jra*g.icells, base + jrb*g.icells, base + (jra + 1)*g.icells, base + (jrb + 1)*g.icells,
                         base + (jra + 1 == M ? 0 : jra + 1)*g.icells, base + (jrb + 1 == M ? 0 : jrb + 1)*g.icells};
@@ -149,12 +151,20 @@ namespace
                     z[q].x = Pa[x]; z[q].y = Pb[x];
                 }
                 #pragma unroll
-                for (int q = 0; q < RU; ++q) { z[q].x = TF(double(z[q].x) - m); z[q].y = TF(double(z[q].y) - m); }
+                for (int q = 0; q < RU; ++q)
+                {
+                    z[q].x = TF(double(z[q].x) - m);
+                    z[q].y = pair ? TF(double(z[q].y) - m) : TF(0);
+                }
             }
             else
             {
                 #pragma unroll
-                for (int q = 0; q < RU; ++q) z[q] = rhs(min(x0 + q*L, n - 1));
+                for (int q = 0; q < RU; ++q)
+                {
+                    z[q] = rhs(min(x0 + q*L, n - 1));
+                    if (!pair) z[q].y = TF(0);
+                }
             }
             #pragma unroll
             for (int q = 0; q < RU; ++q)
@@ -310,6 +320,7 @@ namespace
                     const int kx = idx >> psh;
                     T* Sr = rows + (idx & (RP - 1))*stride;
                     T xa = va[q], xb = vb[q];
+                    if (j0 + 2*(idx & (RP - 1)) + 1 >= M) { xb.x = TF(0); xb.y = TF(0); }   // an odd last row
                     if (kx == 0 || 2*kx == n) { xa.y = TF(0); xb.y = TF(0); }   // real bins of a real row
                     T z; z.x = xa.x - xb.y; z.y = xa.y + xb.x;
                     Sr[lpad(kx)] = z;
