@@ -676,7 +676,8 @@ namespace
             return fail(MHH_EINVAL, "the fused time-step limits cover the default boundary only");
         // plane-ring kernel; with `limits` also the CFL and dnmul maxima
         const int nti = (g.itot + VTX - 1)/VTX, ntj = (g.jtot + VTY - 1)/VTY;
-        const int kchunk = c->visc_kchunk > 0 ? c->visc_kchunk : march_kchunk(c, nti*ntj, g.ktot, MARCH_LEAST_VISC);
+        const int kchunk = c->visc_kchunk > 0 ? c->visc_kchunk
+                         : march_kchunk(c, nti*ntj, g.ktot, MARCH_LEAST_VISC, visc_most(sizeof(TF) == 8, lim, sfc, ms));
         const int nkc = (g.ktot + kchunk - 1)/kchunk;
         // the wall mirror and the cyclic update of the pass done inside it where
         // every ghost column is one periodic image and kgc = 1

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <climits>
 #include <cstdint>
 #include <map>
 #include <string>
@@ -221,30 +222,45 @@ namespace mhh
     // Levels per block of the k-marching plane-ring kernels: 64, or fewer
     // on small grids, so that a launch still has about 4 blocks per CU (each
     // chunk reads a few levels past its ends again; 8 levels is the floor), and
-    // down to 2 levels while the launch has fewer than `least` blocks: a level
-    // costs a block a trip to memory, and reading the ends again costs little
-    // where most of the chip is idle.  least: a block per CU for the tendency
-    // passes, whose chunks begin with a dozen planes (32^3 FP32, 32 blocks of 8 levels:
-    // 27.6 us, 128 of 2: 14.5; but 90 x 75 x 60 FP64, 304 blocks of 8, gains nothing
-    // from 4, and 150 x 100 x 75 FP32, 750 of 8, loses a fifth), four for the
-    // viscosity (32^3 13.5 and 8.5 us, 90 x 75 x 60 17.8 and 13.8).  The results do not depend on it.
+    // down to 2 levels while the launch has fewer than `least` blocks and the
+    // halved chunks give at most `most`: a level costs a block a trip to memory,
+    // and reading the ends again costs little where most of the chip is idle.
+    // The results do not depend on it.
+    // least: a block per CU for the tendency passes, whose chunks begin with a
+    // dozen planes (32^3 FP32, 32 blocks of 8 levels: 27.6 us, 128 of 2: 14.5; but
+    // 90 x 75 x 60 FP64, 304 blocks of 8, gains nothing from 4, and 150 x 100 x 75
+    // FP32, 750 of 8, loses a fifth), four for the viscosity (32^3 13.5 and 8.5 us).
     constexpr int MARCH_LEAST_TEND = 256, MARCH_LEAST_VISC = 1024;
-    inline int march_kchunk(int ntiles_xy, int ktot, int least)
+    inline int march_kchunk(int ntiles_xy, int ktot, int least, int most)
     {
         auto blocks = [&](int kc) { return static_cast<long>(ntiles_xy)*((ktot + kc - 1)/kc); };
         int kc = 64;
         while (kc > 8 && blocks(kc) < 1024) kc /= 2;
-        while (kc > 2 && blocks(kc) < least) kc /= 2;
+        while (kc > 2 && blocks(kc) < least && blocks(kc/2) <= most) kc /= 2;
         return kc;
     }
 
-    // The same choice for a context: in a batch recording the launch is
+    // most, for the viscosity: the blocks of its kernels that run at once (their
+    // VGPRs leave 8 on a CU in FP32, 7 with Mason damping, 5 with the limits, and 4 in FP64
+    // with the surface model or the limits).  Beyond that the short chunks run in a second
+    // round, which costs what they saved: 128 x 128 x 96 FP64 with the surface
+    // model, 768 blocks of 8 levels 24.7 us, 1536 of 4 27.8; 96 x 96 x 64, 768
+    // of 4 14.5, 1536 of 2 17.9; 256 x 160 x 24 FP32 with Mason damping, 960 of 4
+    // 12.8, 1920 of 2 15.6.  FP64 without a surface model has 5 on a CU and
+    // gains up to 6 (128 x 128 x 96 20.5 us by 768, 19.0 by 1536; 192 x 144 x 64 22.7 by 864, 24.2 by 1728).
+    inline int visc_most(bool fp64, bool limits, bool sfc, bool mason)
+    {
+        if (fp64) return sfc || limits ? 1024 : 1536;
+        return limits ? 1280 : sfc && mason ? 1792 : 2048;
+    }
+
+    // While a context records into a batch its marching kernels run
     // merged with the other members', which fill the chip together, so each
     // member marches 32 levels per chunk (64-member ensemble step: 8.63 ms,
     // against 9.19 with 64 levels and 8.87 with 16).
-    inline int march_kchunk(const mhh_ctx* c, int ntiles_xy, int ktot, int least)
+    inline int march_kchunk(const mhh_ctx* c, int ntiles_xy, int ktot, int least, int most = INT_MAX)
     {
-        return c->rec ? 32 : march_kchunk(ntiles_xy, ktot, least);
+        return c->rec ? 32 : march_kchunk(ntiles_xy, ktot, least, most);
     }
 
     // Max-reductions: each thread folds a chunk of RED_KCHUNK levels of its

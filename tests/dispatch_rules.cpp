@@ -1,0 +1,23 @@
+// Answers of the library's dispatch rules, one line per line of standard input:
+//   visc TILES KTOT FP64 LIMITS SURFACE MASON   levels per block of the viscosity kernel
+#include <iostream>
+#include <sstream>
+
+#include "mhh_internal.h"
+
+int main()
+{
+    std::string line, what;
+    while (std::getline(std::cin, line))
+    {
+        std::istringstream in(line);
+        in >> what;
+        if (what == "visc")
+        {
+            int tiles, ktot, fp64, limits, sfc, mason;
+            in >> tiles >> ktot >> fp64 >> limits >> sfc >> mason;
+            std::cout << mhh::march_kchunk(tiles, ktot, mhh::MARCH_LEAST_VISC, mhh::visc_most(fp64, limits, sfc, mason));
+        }
+        std::cout << "\n";
+    }
+}

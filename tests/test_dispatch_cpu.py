@@ -1,0 +1,40 @@
+"""The dispatch rules of the library on the CPU: a small program with the rules'
+own headers answers for given sizes, so a change of a rule that sends a size
+elsewhere is seen without a GPU.
+
+Viscosity chunks: a launch of the viscosity kernel halves its chunks of levels
+only while the halved chunks still run at once, which is what it gains by
+(times in us on an MI355X: 128 x 128 x 96 FP64 with the surface model 24.7 with
+8 levels per block, 27.8 with 4).
+"""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rules") / "dispatch_rules")
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-host-only", "-O1", "-std=c++17",
+                    "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "microhh_amd", "csrc"), "-x", "hip",
+                    os.path.join(ROOT, "tests", "dispatch_rules.cpp"), "-o", exe], check=True)
+
+    def ask(*lines):
+        r = subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True)
+        return r.stdout.split("\n")[:len(lines)]
+    return ask
+
+
+@pytest.mark.parametrize("itot,jtot,ktot,fp64,limits,sfc,mason,levels", [
+    (128, 128, 96, 1, 0, 1, 1, 8), (150, 100, 75, 1, 0, 1, 1, 8), (96, 96, 64, 1, 0, 1, 1, 4),
+    (90, 75, 61, 1, 0, 1, 0, 4), (32, 32, 32, 1, 0, 1, 1, 2),
+    (128, 128, 96, 1, 0, 0, 0, 4), (192, 144, 64, 1, 0, 0, 0, 8), (200, 160, 20, 1, 0, 0, 0, 4),
+    (128, 128, 96, 1, 1, 0, 0, 8), (256, 160, 24, 0, 0, 1, 1, 4), (150, 100, 75, 0, 0, 1, 1, 4),
+    (320, 256, 12, 0, 0, 1, 1, 4), (160, 128, 80, 0, 0, 0, 0, 4), (32, 32, 32, 0, 0, 0, 0, 2),
+    (512, 512, 256, 1, 0, 0, 0, 64)])
+def test_viscosity_chunks(rules, itot, jtot, ktot, fp64, limits, sfc, mason, levels):
+    tiles = ((itot + 63) // 64) * ((jtot + 3) // 4)
+    assert rules(f"visc {tiles} {ktot} {fp64} {limits} {sfc} {mason}") == [str(levels)]
