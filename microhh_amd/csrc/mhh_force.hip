@@ -70,8 +70,8 @@ namespace
         }
         mhh::Timer _t(c, "force");
         double* part = c->force_buf + 1;
-        MHH_CHECK(plane_sums<TF>(c, static_cast<const TF*>(c->f.u), static_cast<const TF*>(c->f.ut), g.kstart, g.ktot,
-                                 part));
+        const Plane_fields<TF> uv{{static_cast<const TF*>(c->f.u), static_cast<const TF*>(c->f.ut)}};
+        MHH_CHECK(plane_sums<TF>(c, uv, 2, g.kstart, g.ktot, part));
         fixed_flux_force_g<<<1, FT, 0, c->stream>>>(part, c->force_buf, c->force_dz + g.kstart, nchunk, g.ktot,
                                                     static_cast<double>(g.itot)*g.jtot, uflux, utrans, 1./dt,
                                                     c->h_zh[g.kend]);

@@ -348,15 +348,16 @@ namespace mhh
     // Surface layer and buffer state (mhh_surface.hip).
     void surface_free(mhh_ctx* ctx);
 
-    // Plane sums and means (mhh_stats.hip), FP64 sums over the interior in a
-    // fixed order.  plane_sums: partial sums of the levels k0 .. k0+nk-1 of a
-    // and, unless null, b, part[(field*nk + level)*plane_chunks + chunk].
-    // mean_profile: the horizontal mean of every level (kcells values,
-    // src/field3d_operators.cxx:46-66) into the device array prof; part:
-    // kcells*plane_chunks values of scratch.
+    // Plane sums and means (mhh_stats.hip) of nf fields in one pass, FP64 sums
+    // over the interior in a fixed order.  plane_sums: partial sums of the levels
+    // k0 .. k0+nk-1, part[(field*nk + level)*plane_chunks + chunk].
+    // mean_profiles: the horizontal means of every level
+    // (src/field3d_operators.cxx:46-66) into the device array
+    // prof[field*kcells + level]; part: nf*kcells*plane_chunks values of scratch.
+    template<typename TF> struct Plane_fields { const TF* a[3 + MHH_MAX_SCALARS]; };
     int plane_chunks(const Gd& g);
-    template<typename TF> int plane_sums(mhh_ctx* c, const TF* a, const TF* b, int k0, int nk, double* part);
-    template<typename TF> int mean_profile(mhh_ctx* c, const TF* fld, double* part, double* prof);
+    template<typename TF> int plane_sums(mhh_ctx* c, const Plane_fields<TF>& f, int nf, int k0, int nk, double* part);
+    template<typename TF> int mean_profiles(mhh_ctx* c, const Plane_fields<TF>& f, int nf, double* part, double* prof);
 }
 
 #define MHH_CHECK(call) do { int _rc = (call); if (_rc) return _rc; } while (0)

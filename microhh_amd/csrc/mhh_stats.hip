@@ -19,11 +19,10 @@ namespace
     // blocks to fill the chip: at 768 x 384 x 256 FP64 one block per level took
     // 624 us per field (1.0 TB/s), the chunks 240 us for two (5.0 TB/s).
     template<typename TF>
-    __global__ void __launch_bounds__(MT) plane_part_g(const TF* __restrict__ a, const TF* __restrict__ b,
-                                                       double* __restrict__ part, int k0, int rows, Gd g)
+    __global__ void __launch_bounds__(MT) plane_part_g(Plane_fields<TF> f, double* __restrict__ part, int k0, int rows, Gd g)
     {
         __shared__ double s[MT/64];
-        const TF* __restrict__ fld = blockIdx.z ? b : a;
+        const TF* __restrict__ fld = f.a[blockIdx.z];
         const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
         const TF* __restrict__ lev = fld + static_cast<size_t>(k0 + blockIdx.y)*g.ijcells + g.istart
                                    + static_cast<size_t>(g.jstart)*g.icells;
@@ -51,7 +50,8 @@ namespace
                 = (s[0] + s[1]) + (s[2] + s[3]);
     }
 
-    // The means of the levels from their partial sums, one thread per level.
+    // The means of the levels from their partial sums, one thread per level
+    // of a field (nk: of all fields).
     __global__ void __launch_bounds__(64) plane_fold_g(const double* __restrict__ part, double* __restrict__ prof,
                                                        int nchunk, int nk, double npoints)
     {
@@ -144,29 +144,29 @@ namespace mhh
     }
 
     template<typename TF>
-    int plane_sums(mhh_ctx* c, const TF* a, const TF* b, int k0, int nk, double* part)
+    int plane_sums(mhh_ctx* c, const Plane_fields<TF>& f, int nf, int k0, int nk, double* part)
     {
         const Gd& g = c->gd;
         const int nchunk = plane_chunks(g), rows = (g.jtot + nchunk - 1)/nchunk;
-        plane_part_g<TF><<<dim3(nchunk, nk, b ? 2 : 1), MT, 0, c->stream>>>(a, b, part, k0, rows, g);
+        plane_part_g<TF><<<dim3(nchunk, nk, nf), MT, 0, c->stream>>>(f, part, k0, rows, g);
         return check_launch("plane_sums");
     }
 
     template<typename TF>
-    int mean_profile(mhh_ctx* c, const TF* fld, double* part, double* prof)
+    int mean_profiles(mhh_ctx* c, const Plane_fields<TF>& f, int nf, double* part, double* prof)
     {
         const Gd& g = c->gd;
         mhh::Timer _t(c, "mean_profile");
-        MHH_CHECK(plane_sums<TF>(c, fld, nullptr, 0, g.kcells, part));
-        plane_fold_g<<<(g.kcells + 63)/64, 64, 0, c->stream>>>(part, prof, plane_chunks(g), g.kcells,
-                                                               static_cast<double>(g.itot)*g.jtot);
+        MHH_CHECK(plane_sums<TF>(c, f, nf, 0, g.kcells, part));
+        plane_fold_g<<<(nf*g.kcells + 63)/64, 64, 0, c->stream>>>(part, prof, plane_chunks(g), nf*g.kcells,
+                                                                  static_cast<double>(g.itot)*g.jtot);
         return check_launch("mean_profile");
     }
 
-    template int plane_sums<double>(mhh_ctx*, const double*, const double*, int, int, double*);
-    template int plane_sums<float>(mhh_ctx*, const float*, const float*, int, int, double*);
-    template int mean_profile<double>(mhh_ctx*, const double*, double*, double*);
-    template int mean_profile<float>(mhh_ctx*, const float*, double*, double*);
+    template int plane_sums<double>(mhh_ctx*, const Plane_fields<double>&, int, int, int, double*);
+    template int plane_sums<float>(mhh_ctx*, const Plane_fields<float>&, int, int, int, double*);
+    template int mean_profiles<double>(mhh_ctx*, const Plane_fields<double>&, int, double*, double*);
+    template int mean_profiles<float>(mhh_ctx*, const Plane_fields<float>&, int, double*, double*);
 }
 
 extern "C" int mhh_fields_check(mhh_ctx* c, double* mom, double* tke, double* mass)
