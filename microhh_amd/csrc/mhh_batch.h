@@ -84,6 +84,16 @@ namespace mhh
         return check_launch("batched launch");
     }
 
+    // Bytes of an argument buffer that is made for `size` bytes.  Twice as many: the
+    // substeps of a step differ (12 members FP32: 47, 19, 64 and 67 kB), and a buffer that
+    // has to grow in the middle of a step waits for the GPU and is allocated
+    // anew (1.1 to 1.6 ms of a first step of 3.5).
+    inline size_t batch_capacity(size_t size)
+    {
+        const size_t cap = (2*size + 4095)/4096*4096;
+        return cap > 65536 ? cap : 65536;
+    }
+
     // Appends one launch to the sequence of the recording context (mhh_batch.hip).
     void batch_record(mhh_ctx* c, Batch_fn fn, const void* k, size_t size, dim3 grid, dim3 block, size_t lds);
     // A device double that the end of the recording copies to *dst (the

@@ -63,6 +63,7 @@ namespace
     using mhh::fail;
     using mhh::check_hip;
     using mhh::Batch_slot;
+    using mhh::batch_capacity;
 
     constexpr size_t ALIGN = 16;
     size_t align_up(size_t x, size_t a) { return (x + a - 1)/a*a; }
@@ -197,7 +198,7 @@ namespace
                 victim->d = nullptr;
                 victim->cap = 0;
             }
-            const size_t cap = std::max<size_t>(align_up(blob.size(), 4096), 65536);
+            const size_t cap = batch_capacity(blob.size());
             MHH_CHECK(check_hip(hipMalloc(&victim->d, cap), "hipMalloc(batch arguments)"));
             victim->cap = cap;
         }
@@ -207,7 +208,7 @@ namespace
             if (b->h_stage) (void)hipHostFree(b->h_stage);
             b->h_stage = nullptr;
             b->h_cap = 0;
-            const size_t cap = std::max<size_t>(align_up(blob.size(), 4096), 65536);
+            const size_t cap = batch_capacity(blob.size());
             MHH_CHECK(check_hip(hipHostMalloc(reinterpret_cast<void**>(&b->h_stage), cap, hipHostMallocDefault),
                                 "hipHostMalloc(batch staging)"));
             b->h_cap = cap;

@@ -1,9 +1,10 @@
 // Answers of the library's dispatch rules, one line per line of standard input:
 //   visc TILES KTOT FP64 LIMITS SURFACE MASON   levels per block of the viscosity kernel
+//   batch SIZE                                  bytes of an argument buffer made for SIZE bytes
 #include <iostream>
 #include <sstream>
 
-#include "mhh_internal.h"
+#include "mhh_batch.h"
 
 int main()
 {
@@ -17,6 +18,12 @@ int main()
             int tiles, ktot, fp64, limits, sfc, mason;
             in >> tiles >> ktot >> fp64 >> limits >> sfc >> mason;
             std::cout << mhh::march_kchunk(tiles, ktot, mhh::MARCH_LEAST_VISC, mhh::visc_most(fp64, limits, sfc, mason));
+        }
+        else if (what == "batch")
+        {
+            size_t size;
+            in >> size;
+            std::cout << mhh::batch_capacity(size);
         }
         std::cout << "\n";
     }

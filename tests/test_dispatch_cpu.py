@@ -6,6 +6,11 @@ Viscosity chunks: a launch of the viscosity kernel halves its chunks of levels
 only while the halved chunks still run at once, which is what it gains by
 (times in us on an MI355X: 128 x 128 x 96 FP64 with the surface model 24.7 with
 8 levels per block, 27.8 with 4).
+
+Argument buffers of a batch: the first substep of a step records fewer launches
+than the others (12 members FP32: 46,848 bytes of arguments, then up to 66,960), and
+a buffer that was made for it holds the others too; one that grows in the middle
+of a step waits for the GPU.
 """
 import os
 import subprocess
@@ -38,3 +43,8 @@ def rules(tmp_path_factory):
 def test_viscosity_chunks(rules, itot, jtot, ktot, fp64, limits, sfc, mason, levels):
     tiles = ((itot + 63) // 64) * ((jtot + 3) // 4)
     assert rules(f"visc {tiles} {ktot} {fp64} {limits} {sfc} {mason}") == [str(levels)]
+
+
+@pytest.mark.parametrize("first,largest", [(46848, 66960), (4 * 46848, 4 * 66960), (1, 65536)])
+def test_batch_arguments_fit_what_a_step_needs(rules, first, largest):
+    assert int(rules(f"batch {first}")[0]) >= largest
