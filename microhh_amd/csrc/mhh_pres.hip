@@ -809,15 +809,18 @@ namespace
     // of the spectrum, TC the arithmetic type of the sweep (double in the mixed
     // mode).
     //
-    // What bounds it: on large grids the bytes (768 x 384 x 256 FP64: 0.57 ms, the
-    // spectrum twice in and out and the two tables), on small ones the chain
+    // What bounds it: on large grids the bytes (768 x 384 x 256 FP64: 0.52 ms, 5.3
+    // TB/s of the spectrum twice in and out and the two tables; 0.55 ms with the
+    // blocks of 32 modes dealt to the XCDs in turn), on small ones the chain
     // over the levels, a multiply-add each if a level's values have arrived.
     // The loads of TRI_G levels are in flight while the TRI_G before them are
-    // eliminated: 32^3 FP32 7.8 us, 90 x 75 x 60 FP64 15.1, 256 x 192 x 96 mixed
-    // 27, 240 x 180 x 120 FP64 46 (15.5, 36.8, 61.7 and 113 with one level per trip
-    // to memory).  LDSB: the eliminated right-hand side stays in the wave's LDS
-    // column (K x 64 words) for the back substitution, so the spectrum is read
-    // and written once.  Only for columns of at most TRI_LDS bytes, five waves
+    // eliminated: 32^3 FP32 7.8 us, 90 x 75 x 60 FP64 14.8, 256 x 192 x 96 mixed
+    // 25, 240 x 180 x 120 FP64 43 (15.5, 35.5, 58 and 112 with one level per trip
+    // to memory).  That form, 64 modes per wave, was faster on two of 16 sizes, both 513 x 320
+    // modes in FP64 (96 levels 188 us, 210 now; 320 levels 695 and 758).  LDSB: the eliminated
+    // right-hand side stays in the wave's LDS column (K x 64 words) for the
+    // back substitution, so the spectrum is read and written once.  Only for
+    // columns of at most TRI_LDS bytes, five waves
     // on a CU: with longer ones too few waves are in flight (1024 x 1024 x 192
     // mixed, 48 KB: 36.5 against 35.0 ms per step; 768 x 384 x 256 FP64, 128 KB:
     // 24.3 against 22.0), with shorter ones the saved trip shows (256 x 192 x 96
@@ -835,7 +838,11 @@ namespace
         TF* col = reinterpret_cast<TF*>(smem_raw) + threadIdx.x;    // LDSB: level k at col[64 k]
         const int M = g.jtot, K = g.ktot;
         const int nmodes = nx*M;
-        const int r0 = bid_.x*64 + static_cast<int>(threadIdx.x);
+        // every XCD takes a contiguous range of modes: a level of its share is then
+        // one run of memory, and the tables of modes ky and M - ky meet in one L2
+        const int tile = xcd_tile(bid_.x, bid_.nx);
+        if (64*tile >= 2*nmodes) return;
+        const int r0 = 64*tile + static_cast<int>(threadIdx.x);
         const bool active = r0 < 2*nmodes;
         const int r = active ? r0 : 2*nmodes - 1;
         const int mode = r >> 1;
@@ -1725,7 +1732,7 @@ namespace
     int tdma(mhh_ctx* c, cplx<TF>* C, const Pres_tables<TC>& t, int nx, bool skip_mean)
     {
         const Gd& g = c->gd;
-        const int nb = (2*nx*g.jtot + 63)/64;
+        const int nb = xcd_blocks((2*nx*g.jtot + 63)/64);
         const size_t lds = sizeof(TF)*64*static_cast<size_t>(g.ktot);
         {
             mhh::Timer _t(c, "tdma");
