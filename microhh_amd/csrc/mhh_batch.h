@@ -102,13 +102,22 @@ namespace mhh
     // Device memory that recorded launches may use, freed after they ran.
     void batch_defer_free(mhh_ctx* c, void* ptr);
 
+    // Records a kernel that runs as a functor only in a batch (its form outside
+    // one is a kernel of its own).
     template<typename K>
-    void launch(mhh_ctx* c, const K& k, dim3 grid, dim3 block, size_t lds = 0)
+    void record(mhh_ctx* c, const K& k, dim3 grid, dim3 block, size_t lds = 0)
     {
         static_assert(std::is_trivially_copyable<K>::value, "kernel functors are copied bytewise");
         static_assert(alignof(K) <= 16, "kernel functors are stored at 16-byte boundaries");
         if (grid.x == 0 || grid.y == 0 || grid.z == 0) return;
-        if (c->rec) { batch_record(c, &batch_launch<K>, &k, sizeof(K), grid, block, lds); return; }
+        batch_record(c, &batch_launch<K>, &k, sizeof(K), grid, block, lds);
+    }
+
+    template<typename K>
+    void launch(mhh_ctx* c, const K& k, dim3 grid, dim3 block, size_t lds = 0)
+    {
+        if (c->rec) return record(c, k, grid, block, lds);
+        if (grid.x == 0 || grid.y == 0 || grid.z == 0) return;
         if constexpr (K::MINB > 0) one_g<K><<<grid, block, lds, c->stream>>>(k);
         else one_g0<K><<<grid, block, lds, c->stream>>>(k);
     }

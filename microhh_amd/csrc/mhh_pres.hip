@@ -1786,7 +1786,7 @@ namespace
         const TF* u = static_cast<const TF*>(c->f.u); const TF* v = static_cast<const TF*>(c->f.v);
         const TF* w = static_cast<const TF*>(c->f.w); const TF* ut = static_cast<const TF*>(c->f.ut);
         const TF* vt = static_cast<const TF*>(c->f.vt); const TF* wt = static_cast<const TF*>(c->f.wt);
-#define MHH_XF(MODE) do { if (c->rec) launch(c, fft_x_fwd_wave_k<TF, R, MODE>{P, C, tw, g, c->pm_mean, c->pm_part, \
+#define MHH_XF(MODE) do { if (c->rec) record(c, fft_x_fwd_wave_k<TF, R, MODE>{P, C, tw, g, c->pm_mean, c->pm_part, \
                 u, v, w, ut, vt, wt, p.dzi, p.rhoref, p.rhorefh, dxi, dyi, dti, cpx, packed}, grd, blk); \
             else fft_x_fwd_wave_direct<TF, R, MODE><<<grd, blk, 0, c->stream>>>(P, C, tw, g, c->pm_mean, c->pm_part, \
                 u, v, w, ut, vt, wt, p.dzi, p.rhoref, p.rhorefh, dxi, dyi, dti, cpx, packed); } while (0)

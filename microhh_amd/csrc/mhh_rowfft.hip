@@ -433,7 +433,7 @@ namespace mhh
                 auto go = [&](auto dc) {
                     constexpr bool D = decltype(dc)::value;
                     if (c->rec)
-                        launch(c, row_x_fwd_k<TF, V, A, D>{C, p, t2, P, c->pm_mean, u, v, w, ut, vt, wt, pr.dzi, pr.rhoref,
+                        record(c, row_x_fwd_k<TF, V, A, D>{C, p, t2, P, c->pm_mean, u, v, w, ut, vt, wt, pr.dzi, pr.rhoref,
                                                            pr.rhorefh, dxi, dyi, dti, nw, xg, g}, xg.nb, 64*nw, lds);
                     else
                         row_x_fwd_direct<TF, V, A, D><<<xg.nb, 64*nw, lds, c->stream>>>(C, p, t2, P, c->pm_mean, u, v, w, ut,
