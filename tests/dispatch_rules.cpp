@@ -1,10 +1,13 @@
 // Answers of the library's dispatch rules, one line per line of standard input:
 //   visc TILES KTOT FP64 LIMITS SURFACE MASON   levels per block of the viscosity kernel
+//   row N ROWS                                  lanes per row, values per lane and butterflies of a
+//                                               launch over ROWS rows of N points, or "none"
 //   batch SIZE                                  bytes of an argument buffer made for SIZE bytes
 #include <iostream>
 #include <sstream>
 
 #include "mhh_batch.h"
+#include "mhh_rowfft.h"
 
 int main()
 {
@@ -18,6 +21,15 @@ int main()
             int tiles, ktot, fp64, limits, sfc, mason;
             in >> tiles >> ktot >> fp64 >> limits >> sfc >> mason;
             std::cout << mhh::march_kchunk(tiles, ktot, mhh::MARCH_LEAST_VISC, mhh::visc_most(fp64, limits, sfc, mason));
+        }
+        else if (what == "row")
+        {
+            int n;
+            long long rows;
+            mhh::Row_plan p;
+            in >> n >> rows;
+            if (!mhh::make_row_plan(n, rows, p)) std::cout << "none";
+            else std::cout << (1 << p.lsh) << " " << p.vals << " " << (p.arith == mhh::ROW_DIRECT ? "direct" : "radix8");
         }
         else if (what == "batch")
         {

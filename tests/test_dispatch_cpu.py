@@ -7,6 +7,10 @@ only while the halved chunks still run at once, which is what it gains by
 (times in us on an MI355X: 128 x 128 x 96 FP64 with the surface model 24.7 with
 8 levels per block, 27.8 with 4).
 
+Transforms by lane groups: the plans that the GPU tests of tests/test_gpu_rowfft.py name
+for their grids, so that a change of the rule cannot take them off the narrow
+groups unseen, and the lengths without a plan.
+
 Argument buffers of a batch: the first substep of a step records fewer launches
 than the others (12 members FP32: 46,848 bytes of arguments, then up to 66,960), and
 a buffer that was made for it holds the others too; one that grows in the middle
@@ -48,3 +52,28 @@ def test_viscosity_chunks(rules, itot, jtot, ktot, fp64, limits, sfc, mason, lev
 @pytest.mark.parametrize("first,largest", [(46848, 66960), (4 * 46848, 4 * 66960), (1, 65536)])
 def test_batch_arguments_fit_what_a_step_needs(rules, first, largest):
     assert int(rules(f"batch {first}")[0]) >= largest
+
+
+def test_plans_of_the_gpu_tests(rules):
+    from tests.test_gpu_rowfft import FALLBACK, NARROW, NARROW32
+    for itot, jtot, ktot, x, y in NARROW + NARROW32:
+        got = rules(f"row {itot} {(jtot + 1) // 2 * ktot}", f"row {jtot} {(itot // 2 + 1) * ktot}")
+        for want, answer in zip((x, y), got):
+            if want == "none":
+                assert answer == "none"
+            else:
+                lanes, values, arith = answer.split()
+                assert f"{lanes} {arith}" == want, (itot, jtot, ktot)
+    for itot, jtot, ktot in FALLBACK:
+        assert "none" in rules(f"row {itot} 100", f"row {jtot} 100")
+
+
+def test_lengths_without_a_plan(rules):
+    def rest(n):
+        for q in (2, 3, 5, 7, 11, 13):
+            while n % q == 0:
+                n //= q
+        return n
+    smooth = [n for n in range(1, 2049) if rest(n) == 1]
+    none = [n for n, a in zip(smooth, rules(*[f"row {n} 1000" for n in smooth])) if a == "none"]
+    assert none[:2] == [1, 1050] and len([n for n in smooth if n > 1024]) == 105 and len(none) == 1 + 55

@@ -1,7 +1,7 @@
 """Pressure projection at transform lengths that have specialised kernels
 (128, 256 and 512 points along x and y, with 7, 9 and 17 levels) against the
 oracle, and the
-specialised kernels against the general LDS engine (MHH_FFT_GENERIC=1) on the
+specialised kernels against the general transforms (MHH_FFT_GENERIC=1) on the
 same inputs.  FP64; tolerance 1e-12 normwise, as for every pressure test.
 """
 import os
@@ -126,12 +126,14 @@ def test_float_specialised_matches_general_engine(prec, n):
         assert err < 1e-5, f"{name}: {err:.3e}"
 
 
-# Lengths of the general engine's three kernel instances: the fast engine
-# with 16 values per lane and pass (96 = 4 8 3, 768 = 4 8 8 3), the wide one
-# (1000 = 8 5 5 5: radix-5 passes of 200 butterflies, 4 per lane) and the
-# ping-pong fallback (a radix-7 pass, 56 = 8 7; 1300 = 4 5 5 13 with a
-# radix-13 pass and a radix-4 pass of 325 butterflies).
-@pytest.mark.parametrize("itot,jtot", [(96, 768), (1000, 12), (56, 1300)], ids=["fast", "wide", "pingpong"])
+# The instances of the general transforms (MHH_FFT_GENERIC): lane groups with 16
+# values per lane and radices 8, 4, 2, 3, 5 (96 = 4 8 3, 768 = 4 8 8 3), with 32
+# values (1000 = 8 5 5 5: radix-5 passes of 200 butterflies, 4 per lane), with
+# butterflies by definition (56 = 8 7; 1300 = 4 5 5 13 with a radix-13 pass and a
+# radix-4 pass of 325 butterflies), and the ping-pong transform in two row
+# buffers of the lengths without a plan (1050 = 2 3 5 5 7, 1078 = 2 7 7 11).
+@pytest.mark.parametrize("itot,jtot", [(96, 768), (1000, 12), (56, 1300), (1050, 9), (8, 1078)],
+                         ids=["values16", "values32", "direct", "pingpong-x", "pingpong-y"])
 def test_pres_general_engine_instances(itot, jtot):
     from tests.golden.make_golden import make_inputs
     p, i = make_inputs(dict(itot=itot, jtot=jtot, ktot=6, stretch=True, anelastic=True, dx=50.0, dy=40.0,

@@ -1,7 +1,10 @@
 """Transforms by lane groups at the lengths where their plan changes: one to
 several passes, every radix and both kinds of butterflies, rows that do not fill a
-group, odd numbers of rows (a pair with one row), 8 to 64 lanes per row (few and many
-rows), the wide instance (864, 1000, 1200, 1536), and a length without a plan (1050).
+group, odd numbers of rows (a pair with one row), the instance with 32 values
+per lane (864, 1000, 1200, 1536), and a length without a plan (1050).  Few rows take 64
+lanes each; NARROW holds grids with enough rows for 8, 16 and 32 lanes, several
+rows to a wave and a last wave that is partly idle (tests/test_dispatch_cpu.py checks that
+their plans are these).  FALLBACK: x and y transforms of lengths without a plan.
 
 Against the oracle, normwise.  FP64: 1e-12 as for every pressure test.  FP32 and
 mixed: 1e-5, the bound of the FP32 transforms in test_gpu_fft_sizes.py.  Both up to
@@ -10,9 +13,12 @@ the gradient of its largest wave, 2 pi |p| / (n dx), the difference of two
 neighbours is off by a relative eps n / (2 pi) (FP32 2e-5 at 2048 points); the smallest
 eigenvalue, a difference of 1 and cos(2 pi / n), loses digits with n as well, so the same
 factor is used for p.  Plain FP32: its sweeps of up to K = 9 levels amplify roundings
-by at most about K^2, and 81 times 6e-8 is half of 1e-5; long rows are left to the
-mixed mode, since there the rounding of the mean, which plain FP32 carries through
-its transforms, is more than the fluctuations allow in this measure.
+by at most about K^2, and 81 times 6e-8 is half of 1e-5.  On long rows it carries a p that
+is large against its gradient, the mean above all, through its transforms.  A pass of
+radix R sums R products with rounded roots, (R + 2) 2^-24 of the largest value;
+a p has gone through the passes of both lengths forward and inverse, and a tendency takes the
+difference of two p: 4 sum (R + 2) 2^-24 max|p| / spacing, the bound where that is more
+(the sum over the prime factors of both lengths, which is no less than over the radices).
 """
 import pytest
 
@@ -47,6 +53,59 @@ def test_fp64(itot, jtot, ktot):
         assert err < TOL * _longer(itot, jtot), f"{name}: {err:.3e}"
     err = normwise(out["p"][d.kstart - 1:d.kend], ref["p"][d.kstart - 1:d.kend])
     assert err < TOL * _longer(itot, jtot), f"p: {err:.3e}"
+
+
+# itot, jtot, ktot, lanes and butterflies of the x transform, the same of the y transform
+NARROW = [(15, 637, 52, "8 radix8", "64 direct"), (14, 625, 53, "8 direct", "64 radix8"),
+          (600, 15, 55, "64 radix8", "8 radix8"), (600, 13, 55, "64 radix8", "8 direct"),
+          (12, 315, 57, "16 radix8", "64 direct"), (315, 14, 57, "64 direct", "16 direct"),
+          (24, 175, 47, "32 radix8", "64 direct"), (175, 24, 47, "64 direct", "32 radix8")]
+# the same with 9 levels, for plain FP32
+NARROW32 = [(15, 3645, 9, "8 radix8", "none"), (14, 3645, 9, "8 direct", "none"), (12, 1875, 9, "16 radix8", "none"),
+            (24, 945, 9, "32 radix8", "64 direct")]
+
+
+def _passes(*lengths):
+    total = 0
+    for n in lengths:
+        for q in (2, 3, 5, 7, 11, 13):
+            while n % q == 0:
+                n //= q
+                total += q + 2
+    return total
+
+
+def _check(itot, jtot, ktot, precision):
+    import numpy as np
+    from microhh_amd import abi
+    p, i = _case(itot, jtot, ktot)
+    out, uvw = _gpu_pres(p, i, 0.37, generic=True,
+                         precision=dict(fp64=abi.MHH_FP64, fp32=abi.MHH_FP32, mixed=abi.MHH_MIXED)[precision])
+    d, ref = _oracle_pres(p, i, uvw, 0.37)
+    m = interior(d)
+    for name, spacing in (("ut", p["dx"]), ("vt", p["dy"]), ("wt", np.min(i["dz"]))):
+        bound = (TOL if precision == "fp64" else 1e-5) * _longer(itot, jtot)
+        if precision == "fp32":
+            rounding = 4 * _passes(itot, jtot) * 2.0**-24 * np.abs(ref["p"][m]).max() / spacing
+            bound = max(bound, rounding / np.abs(ref[name][m]).max())
+        err = normwise(out[name], ref[name], m)
+        assert err < bound, f"{name}: {err:.3e}, bound {bound:.3e}"
+
+
+@pytest.mark.parametrize("itot,jtot,ktot,precision",
+                         [(*s[:3], q) for s in NARROW for q in ("fp64", "mixed")] + [(*s[:3], "fp32") for s in NARROW32])
+def test_several_rows_per_wave(itot, jtot, ktot, precision):
+    _check(itot, jtot, ktot, precision)
+
+
+# in x with an odd and an even length and an odd number of rows, and in y
+FALLBACK = [(1050, 9, 6), (1485, 7, 6), (6, 1050, 6)]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "mixed"])
+@pytest.mark.parametrize("itot,jtot,ktot", FALLBACK)
+def test_lengths_without_a_plan(itot, jtot, ktot, precision):
+    _check(itot, jtot, ktot, precision)
 
 
 ROWS32 = [(13, 11, 6), (75, 90, 9), (250, 36, 6), (64, 16, 7)]
