@@ -17,7 +17,10 @@ namespace mhh
     {
         int n;
         int npass;
-        int fast;       // nonzero: radices 2, 3, 4, 5, 8 and at most 256 butterflies in every pass
+        // nonzero: radices 2, 3, 4, 5, 8 and at most 256 butterflies in every pass.
+        // These lengths take the codelets, the others sum by definition (two
+        // different roundings, so the line stays where it was drawn)
+        int fast;
         int radix[FFT_MAXPASS];
     };
 

@@ -106,7 +106,7 @@ namespace mhh
         int nb[ROW_MAXPASS];        // butterflies n/R
         int ns[ROW_MAXPASS];        // product of the radices before
         int ts[ROW_MAXPASS];        // twiddle stride n/(ns R)
-        unsigned int mg[ROW_MAXPASS];   // j/ns = (j mg) >> 22 for j < 2048
+        unsigned int mg[ROW_MAXPASS];   // j/ns = (j mg) >> 22 for j < 2048, ns >= 2 (32-bit product)
     };
 }
 

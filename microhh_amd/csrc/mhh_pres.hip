@@ -17,8 +17,9 @@
 //
 // FFT: Stockham autosort with twiddles from a host-computed table: a wave per row
 // for 128, 256 and 512 points (here), lane groups for the other lengths
-// (mhh_rowfft.hip), DFT-as-GEMM for 1024 in the mixed mode (mhh_dft.hip), and the ping-pong engine of mhh_fft.h for the few lengths that have
-// no lane-group plan.
+// (mhh_rowfft.hip), DFT-as-GEMM for 1024 in the mixed mode (mhh_dft.hip), and the
+// ping-pong engine of mhh_fft.h for the lengths that have no lane-group plan (55
+// of the 105 from 1025 to 2048, none below 1050, all above).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>

@@ -10,7 +10,10 @@
 //   ROW_DIRECT  any radix up to 13 by its definition, the sums in the order of
 //               fft_row_pingpong
 // Order and roundings are those of the block-wide engines that the lane groups took
-// over from, so that the projection kept its bits.  Composite radices up to 16
+// over from: built with the compiler of ROCm 7.2, the projection of 42 grids
+// returned the same bits as with those, in FP64, FP32 and the mixed mode.  turn() writes
+// the roundings of the twiddle products out; those inside dft<> are left to
+// contraction, so another compiler may move the last bits.  Composite radices up to 16
 // would save a pass (960 x 500 x 58 FP64 projection 1.26 ms instead of 1.36), but
 // rounding in another order shows: plain FP32 carries the horizontal mean through
 // transforms and sweeps (4e-3 of a velocity after two steps), and the FP64 eddy
@@ -31,7 +34,10 @@ namespace mhh
     constexpr int ROW_VALS = 16, ROW_VALS_WIDE = 32;   // complex values a lane holds in a pass
     enum { ROW_RADIX8 = 0, ROW_DIRECT = 1 };
     enum { ROW_X_FWD, ROW_Y_FWD, ROW_Y_INV, ROW_X_INV };
-    // and butterflies
+    // Butterflies of radix r that a lane holds in a pass: as many as its values allow,
+    // up to a limit.  4 for ROW_RADIX8: 256 on 64 lanes, the most that make_plan
+    // calls fast.  8 for ROW_DIRECT bounds the unrolled code; it is not tuned
+    // (1920 = 4 4 8 3 5 would need ten of radix 3, whose 30 values fit in the 32).
     __host__ __device__ constexpr int row_rounds(int r, int vals, int arith)
     {
         const int most = arith == ROW_DIRECT ? 8 : 4;

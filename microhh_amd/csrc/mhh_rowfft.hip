@@ -9,7 +9,7 @@
 // What bounds them: the memory traffic of one pass over the fields (x, forward)
 // or the spectrum, and on small grids the latency of the passes.  Measured, against
 // the block-wide engine (a wave per row, block barriers between passes) that they
-// replace, bit for bit:
+// replace:
 //   768 x 384 x 256 FP64: forward x 956 us (7 passes over the fields, 4.5 TB/s;
 //     1629), y 382 (416), inverse x 384 (764)
 //   90 x 75 x 60 FP64: 14.3, 7.9, 8.9 us (15.9, 8.9, 13.1)
