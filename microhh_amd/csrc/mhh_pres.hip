@@ -827,6 +827,7 @@ namespace
     // 24.3 against 22.0), with shorter ones the saved trip shows (256 x 192 x 96
     // mixed: 0.94 against 0.96 ms per step).
     constexpr int TRI_G = 16;
+    constexpr int TRI_XCD = 512;
     constexpr size_t TRI_LDS = 32*1024;
 
     template<typename TF, typename TC, bool LDSB>
@@ -839,9 +840,12 @@ namespace
         TF* col = reinterpret_cast<TF*>(smem_raw) + threadIdx.x;    // LDSB: level k at col[64 k]
         const int M = g.jtot, K = g.ktot;
         const int nmodes = nx*M;
-        // every XCD takes a contiguous range of modes: a level of its share is then
-        // one run of memory, and the tables of modes ky and M - ky meet in one L2
-        const int tile = xcd_tile(bid_.x, bid_.nx);
+        // with two blocks per CU or more every XCD takes a contiguous range of modes: a
+        // level of its share is then one run of memory, and the tables of modes ky
+        // and M - ky meet in one L2.  Fewer are dealt to the XCDs in turn (24 x 24 x 300
+        // FP32, 10 blocks: projection 83.0 us, 86.2 in ranges; 128 x 160 x 64 FP64, 325:
+        // 79.0 and 80.3; but 240 x 180 x 120 FP64, 681: 287.7 and 282.1)
+        const int tile = bid_.nx < TRI_XCD ? bid_.x : xcd_tile(bid_.x, bid_.nx);
         if (64*tile >= 2*nmodes) return;
         const int r0 = 64*tile + static_cast<int>(threadIdx.x);
         const bool active = r0 < 2*nmodes;
@@ -1733,7 +1737,7 @@ namespace
     int tdma(mhh_ctx* c, cplx<TF>* C, const Pres_tables<TC>& t, int nx, bool skip_mean)
     {
         const Gd& g = c->gd;
-        const int nb = xcd_blocks((2*nx*g.jtot + 63)/64);
+        const int tiles = (2*nx*g.jtot + 63)/64, nb = tiles < TRI_XCD ? tiles : xcd_blocks(tiles);
         const size_t lds = sizeof(TF)*64*static_cast<size_t>(g.ktot);
         {
             mhh::Timer _t(c, "tdma");
