@@ -256,8 +256,8 @@ namespace mhh
 
     // While a context records into a batch its marching kernels run
     // merged with the other members', which fill the chip together, so each
-    // member marches 32 levels per chunk (64-member ensemble step: 8.63 ms,
-    // against 9.19 with 64 levels and 8.87 with 16).
+    // member marches 32 levels per chunk (64-member ensemble step: 8.30 ms,
+    // against 8.83 with 64 levels and 8.49 with 16).
     inline int march_kchunk(const mhh_ctx* c, int ntiles_xy, int ktot, int least, int most = INT_MAX)
     {
         return c->rec ? 32 : march_kchunk(ntiles_xy, ktot, least, most);
